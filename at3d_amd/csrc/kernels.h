@@ -185,6 +185,27 @@ void launch_sweep_ring(hipStream_t st, const SweepArgs& a, int col0, int ncol, s
 void launch_sweep_preset(hipStream_t st, const SweepArgs& a, bool up, int col0, int ncol);
 // One workgroup per ordinate column col0 .. col0+ncol-1, all levels of its octant.
 void launch_sweep_columns(hipStream_t st, const SweepArgs& a, int col0, int ncol);
+// ---- sweep_chain.hip: point-ordered sweep from per-ordinate records ------
+// Arrays of one state, rows of npts entries per column: in the octant's list
+// order (q while the levels are made), then in the ordinate's level order.
+struct ChainArrays {
+  ushort4* q = nullptr;       // the four corners the characteristic stops on
+  double *u = nullptr, *v = nullptr;   // their face's interpolation factors
+  double* trans = nullptr;    // transmission of the path
+  double* radv = nullptr;     // [nst] planes: source integral along the path, every sweep
+  uint32_t* ptlev = nullptr;  // the point, and its level in the upper half
+  int32_t* order = nullptr;   // its index in the octant's list
+  int* count = nullptr;       // [ncols][npts + 2] work of the level sort
+  size_t plane = 0;           // ncols * npts
+};
+// Bytes per (column, point) of the arrays above.
+constexpr size_t chain_point_bytes(int nst) { return 8 + 3 * 8 + 8 * (size_t)nst + 4 + 4 + 4; }
+// Allows the launches below with npts points (an LDS row of 4 npts bytes);
+// nonzero on failure.
+int sweep_chain_max_lds(int npts);
+void launch_chain_setup(hipStream_t st, const SweepArgs& a, const ChainArrays& c, int ncol);
+// Columns col0 .. col0+ncol-1 with their boundary radiances, all Stokes components.
+void launch_sweep_chain(hipStream_t st, const SweepArgs& a, const ChainArrays& c, int col0, int ncol);
 // Where the surface radiances also go: the boundary entries of the step
 // records of the upwelling columns col0 .. col1-1 (rec null: nowhere else).
 struct BottomRecs {

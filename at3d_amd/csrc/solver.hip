@@ -168,11 +168,15 @@ static SweepArgs sweep_args(const State& s) {
 
 // The level-ordered sweep, where its rings fit, unless its levels are chains
 // of a point or two (periodic grids, whose multi-cell traces depend on the
-// points swept just before): there the point-ordered sweep's lighter levels
-// are faster (16^3 periodic, NMU 8: 22 against 45 ms per iteration).
+// points swept just before): there the point-ordered sweep, whose levels are
+// each ordinate's own, is faster (16^3 periodic, NMU 8: 0.7 against 45 ms per
+// iteration).
 static bool ring_active(const State& s) {
   return s.ring_ok && s.use_ring && !s.force_general && (s.use_ring == 2 || !s.ring_chain);
 }
+
+// The point-ordered sweep from per-ordinate records (ensure_sweep made them).
+static bool chain_active(const State& s) { return !ring_active(s) && !s.force_general && s.chain == 1; }
 
 // The level-ordered sweep: each octant's ring order (its levels, with the
 // hemisphere's boundary points as entries of their own), the SH->DO column
@@ -389,6 +393,10 @@ size_t plan_footprint_bytes(const Plan& p) {
   b += 8 * npts * 4 * 4 + npts;          // sweep order: rank, level, level lists, preset
   b += nang * npts * 16;                 // sweep records
   b += nang * (size_t)p.nz * 4 * 16 + 8 * nptsp * 4 + 8 * (size_t)p.nz * 4 * 8;  // step classes, ring-order extinction
+  bool chain = !p.treeptr.empty();
+  for (int o = 0; o < 8; o++) chain = chain || (p.oct[o].ring_nlev > 0 && (double)npts / p.oct[o].ring_nlev < 4.0);
+  if (chain && npts <= 40960)            // point-ordered sweep from records, with its level lists
+    b += nang * npts * chain_point_bytes(p.nst) + nang * 8 + 8 * npts * 4 * 2;
   b += 8 * nptsp * 4 + 8 * npts * (4 * 4 + 2) + 8 * (npts / 4 + 8) * 20;  // ring layout, face masks, sectors
   if (p.host_medium)
     b += p.ss_off.size() * 4 + p.ss_iph.size() * 4 + p.ss_coef.size() * 4;
@@ -1002,7 +1010,7 @@ static void enqueue_sweeps(State& s, const int* stop = nullptr) {
   SweepArgs a = sweep_args(s);
   a.stop = stop;
   const float albpi = p.d.gndalbedo / acosf(-1.0f);
-  const bool ring = ring_active(s);
+  const bool ring = ring_active(s), chain = chain_active(s);
   // the ring sweep writes the boundary radiances itself; events around its
   // launches time the sweep kernel alone
   // which ring instantiations each hemisphere's columns need
@@ -1033,6 +1041,8 @@ static void enqueue_sweeps(State& s, const int* stop = nullptr) {
       launch_sweep_ring(s.stream, a, 0, s.ndown, s.ring_lds, s.ring_lds_full, fast, full);
     }
     (void)hipEventRecord(s.ev_sweep[1], s.stream);
+  } else if (chain) {
+    launch_sweep_chain(s.stream, a, s.chain_arrays, 0, s.ndown);
   } else {
     launch_sweep_preset(s.stream, a, false, 0, s.ndown);
     launch_sweep_columns(s.stream, a, 0, s.ndown);
@@ -1046,6 +1056,8 @@ static void enqueue_sweeps(State& s, const int* stop = nullptr) {
     SweepArgs a2 = a;
     if (merge_qu) a2.nst = 1;   // the upwelling I columns alone
     launch_sweep_ring(s.stream, a2, s.ndown, p.nang - s.ndown, s.ring_lds, s.ring_lds_full, fast, full);
+  } else if (chain) {
+    launch_sweep_chain(s.stream, a, s.chain_arrays, s.ndown, p.nang - s.ndown);
   } else {
     launch_sweep_preset(s.stream, a, true, s.ndown, p.nang - s.ndown);
     launch_sweep_columns(s.stream, a, s.ndown, p.nang - s.ndown);
@@ -1071,11 +1083,55 @@ static int ensure_point_order(State& s, std::string& err) {
   return AT3D_OK;
 }
 
+// The arrays the active sweep makes on its first use: the point-ordered
+// sweep's level lists and, where an ordinate's radiances fit in LDS (npts <=
+// 40960) and the records in memory, its per-ordinate records.
+static int ensure_sweep(State& s, std::string& err) {
+  if (ring_active(s)) return AT3D_OK;
+  TRY(ensure_point_order(s, err));
+  if (s.chain || s.force_general) return AT3D_OK;
+  const Plan& p = *s.plan;
+  s.chain = -1;
+  int maxlds = 0;
+  HIPCHK(hipDeviceGetAttribute(&maxlds, hipDeviceAttributeMaxSharedMemoryPerBlock, s.device));
+  if ((size_t)p.npts * 4 > (size_t)maxlds || sweep_chain_max_lds(p.npts) != 0) return AT3D_OK;
+  const size_t n = (size_t)p.nang * p.npts;
+  ChainArrays& c = s.chain_arrays;
+  c.plane = n;
+  // one block, the widest arrays first
+  const size_t bytes = n * chain_point_bytes(s.nst) + (size_t)p.nang * 8;
+  char* b = nullptr;
+  if (dev_alloc((void**)&b, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    return AT3D_OK;
+  }
+  s.allocs.emplace_back(b, bytes);
+  s.device_bytes += bytes;
+  auto take = [&](size_t each) {
+    char* q = b;
+    b += n * each;
+    return q;
+  };
+  c.u = reinterpret_cast<double*>(take(8));
+  c.v = reinterpret_cast<double*>(take(8));
+  c.trans = reinterpret_cast<double*>(take(8));
+  c.radv = reinterpret_cast<double*>(take(8 * (size_t)s.nst));
+  c.q = reinterpret_cast<ushort4*>(take(8));
+  c.order = reinterpret_cast<int32_t*>(take(4));
+  c.ptlev = reinterpret_cast<uint32_t*>(take(4));
+  c.count = reinterpret_cast<int*>(b);
+  launch_chain_setup(s.stream, sweep_args(s), c, p.nang);
+  HIPCHK(hipGetLastError());
+  s.chain = 1;
+  return AT3D_OK;
+}
+
 static int run_sweeps(State& s, std::string& err) {
-  if (!ring_active(s)) TRY(ensure_point_order(s, err));
+  TRY(ensure_sweep(s, err));
   // the level-ordered sweep is three launches per pass (and is timed by
-  // events between them); the point-ordered one is replayed from a graph
-  if (!s.use_graph || ring_active(s)) {
+  // events between them), the one from records five; k_sweep_columns is
+  // replayed from a graph
+  if (!s.use_graph || ring_active(s) || chain_active(s)) {
     enqueue_sweeps(s);
     HIPCHK(hipGetLastError());
     return AT3D_OK;
@@ -1174,6 +1230,11 @@ static void enqueue_iteration(State& s) {
   launch_accelerate(s.stream, s.S, s.DS, s.ns, s.nos, s.ld, p.npts, 0.0f, s.ctl, s.nst, s.psh);
 }
 
+// The sweep configuration a captured graph holds.
+static int iteration_key(const State& s) {
+  return (ring_active(s) ? 1 : 0) | (s.force_general ? 2 : 0) | (s.ring_full ? 4 : 0) | (chain_active(s) ? 8 : 0);
+}
+
 // The graph of ITER_BATCH iterations for the NR buffer parity k (0: s.nr is
 // the first buffer), captured on the state's stream.
 static int capture_iterations(State& s, int k, std::string& err) {
@@ -1195,7 +1256,7 @@ static int capture_iterations(State& s, int k, std::string& err) {
     return AT3D_ERR_DEVICE;
   }
   HIPCHK(hipGraphInstantiate(&s.iter_exec[k], s.iter_graph[k], nullptr, nullptr, 0));
-  s.iter_key[k] = (ring_active(s) ? 1 : 0) | (s.force_general ? 2 : 0) | (s.ring_full ? 4 : 0);
+  s.iter_key[k] = iteration_key(s);
   return AT3D_OK;
 }
 
@@ -1216,7 +1277,7 @@ static int state_solve_graph(State& s, int maxiter, std::string& err) {
   HIPCHK(hipMemcpyAsync(s.ctl, &c, sizeof c, hipMemcpyHostToDevice, s.stream));
   const int parity = s.nr == s.nr_buf0 ? 0 : 1;
   s.dosrc_level_order = ring_active(s);
-  const int key = (ring_active(s) ? 1 : 0) | (s.force_general ? 2 : 0) | (s.ring_full ? 4 : 0);
+  const int key = iteration_key(s);
   if (!s.iter_exec[parity] || s.iter_key[parity] != key) TRY(capture_iterations(s, parity, err));
   // every batch runs ITER_BATCH iterations unless the device stops: the
   // host bound only guards against a control block that never moves
@@ -1448,9 +1509,11 @@ int state_solve(State& s, int maxiter, int verbose, std::string& err) {
   }
   // (p is not used past this call: the state's plan changes when it splits)
   if (p.d.splitacc > 0.0f) return solve_split(s, maxiter, verbose, err);
-  // graphs replay the level-ordered sweep; the point-ordered one (grids whose
-  // ring does not fit in LDS, and the test options) iterates from the host
-  if (s.use_iter_graph && !verbose && ring_active(s) && s.iters < maxiter && s.solcrit > p.d.solacc) {
+  // graphs replay the level-ordered sweep and the one from records;
+  // k_sweep_columns (grids beyond both, and the test options) iterates from
+  // the host
+  if (s.iters < maxiter && s.solcrit > p.d.solacc) TRY(ensure_sweep(s, err));
+  if (s.use_iter_graph && !verbose && (ring_active(s) || chain_active(s)) && s.iters < maxiter && s.solcrit > p.d.solacc) {
     TRY(state_solve_graph(s, maxiter, err));
     s.last_solve_graph = true;
     launch_fluxes(s.stream, s.dorad, s.nptsp, s.col_of_ref_d, s.fluxw, s.ndown, p.nang, p.npts, s.fluxes);

@@ -115,6 +115,10 @@ struct State {
   int* ngeneral_d = nullptr;
   int4* sh_tiles = nullptr;
   int n_sh_tiles = 0;
+  // point-ordered sweep from per-ordinate records (sweep_chain.hip), made on
+  // the point-ordered sweep's first use: 0 not yet, 1 ready, -1 not available
+  int chain = 0;
+  ChainArrays chain_arrays;
   bool dosrc_level_order = false;   // layout of dosrc written by the last SH->DO
   // options
   int force_general = 0;  // 1: every point through the general characteristic trace
