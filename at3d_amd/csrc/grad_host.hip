@@ -197,7 +197,7 @@ int state_levis_gradient(State& s, const at3d_deriv_desc& dd, int64_t nrays, con
   }
   GradPlan g;
   {
-    const int rc = build_grad_plan(p, dd, g, err);
+    const int rc = build_grad_plan(p, dd, g, njac > 0, err);
     if (rc) return rc;
   }
   // ---- Jacobian columns: the grid points whose interpolation kernel or sun
@@ -316,8 +316,8 @@ int state_levis_gradient(State& s, const at3d_deriv_desc& dd, int64_t nrays, con
   const size_t o_dip = carve(g.diphasep.size() * 4), o_dextm = carve(g.dextm.size() * 4);
   const size_t o_legp = carve(sp.legp.size() * 4), o_dlegp = carve(dlegp.size() * 4);
   const size_t o_dfj = carve(g.dfj.size() * 4), o_dalbm = carve(g.dalbm.size() * 4);
-  const size_t o_bpo = carve(g.bp_off.size() * 4), o_bpi = carve(g.bp_ip.size() * 4);
-  const size_t o_bpw = carve(g.bp_w.size() * 4), o_alb = carve(p.albedo.size() * 4);
+  const size_t o_sunw = carve((size_t)maxpg * 8), o_len = carve(((size_t)npts + 1) * 4);
+  const size_t o_alb = carve(p.albedo.size() * 4);
   const size_t o_pd = carve(partder.size() * 4), o_dx = carve(doexact.size() * 4);
   // Jacobian
   const size_t o_jw = carve(njac > 0 ? nr * 8 : 0), o_rels = carve(rel_s.size() * 4);
@@ -377,9 +377,6 @@ int state_levis_gradient(State& s, const at3d_deriv_desc& dd, int64_t nrays, con
   HIPCHK(up(o_dlegp, dlegp.data(), dlegp.size() * 4));
   HIPCHK(up(o_dfj, g.dfj.data(), g.dfj.size() * 4));
   HIPCHK(up(o_dalbm, g.dalbm.data(), g.dalbm.size() * 4));
-  HIPCHK(up(o_bpo, g.bp_off.data(), g.bp_off.size() * 4));
-  HIPCHK(up(o_bpi, g.bp_ip.data(), g.bp_ip.size() * 4));
-  HIPCHK(up(o_bpw, g.bp_w.data(), g.bp_w.size() * 4));
   HIPCHK(up(o_alb, p.albedo.data(), p.albedo.size() * 4));
   HIPCHK(up(o_pd, partder.data(), partder.size() * 4));
   HIPCHK(up(o_dx, doexact.data(), doexact.size() * 4));
@@ -498,6 +495,8 @@ int state_levis_gradient(State& s, const at3d_deriv_desc& dd, int64_t nrays, con
   HIPCHK(hipMemsetAsync(B + o_erad, 0, (size_t)npts * 8, s.stream));
   HIPCHK(hipMemsetAsync(B + o_bw, 0, (size_t)npts * 8, s.stream));
   HIPCHK(hipMemsetAsync(B + o_grad, 0, (size_t)numder * maxpg * 8, s.stream));
+  HIPCHK(hipMemsetAsync(B + o_sunw, 0, (size_t)maxpg * 8, s.stream));
+  HIPCHK(hipMemsetAsync(B + o_len, 0, ((size_t)npts + 1) * 4, s.stream));
   AdjArgs A;
   A.r = a;
   A.ss8 = ss8;
@@ -569,11 +568,10 @@ int state_levis_gradient(State& s, const at3d_deriv_desc& dd, int64_t nrays, con
   G.dlegp = reinterpret_cast<float*>(B + o_dlegp);
   G.dfj = reinterpret_cast<float*>(B + o_dfj);
   G.dalbm = reinterpret_cast<float*>(B + o_dalbm);
-  G.bp_off = reinterpret_cast<int32_t*>(B + o_bpo);
-  G.bp_ip = reinterpret_cast<int32_t*>(B + o_bpi);
-  G.bp_w = reinterpret_cast<float*>(B + o_bpw);
+  G.sunw = reinterpret_cast<double*>(B + o_sunw);
+  G.path_len = reinterpret_cast<int32_t*>(B + o_len);
   launch_grad_points(s.stream, G);
-  if (ess) launch_grad_beam(s.stream, G);
+  if (ess) launch_grad_beam(s.stream, G, s.beam, s.gridpos, s.errflag);
   if (njac > 0) {
     JacArgs J;
     J.npix = (int)npix;
@@ -617,7 +615,8 @@ int state_levis_gradient(State& s, const at3d_deriv_desc& dd, int64_t nrays, con
   (void)hipEventElapsedTime(&ms, s.ev_ray[0], s.ev_ray[1]);
   s.adjoint_ms = ms;
   if (ef) {
-    err = (ef & 32)  ? "ADJOINT_INTEGRATE_1RAY: ray crossed too many cells without leaving the grid"
+    err = (ef & 64)  ? "DIRECT_BEAM_AND_PATHS_PROP: ray left the property grid"
+          : (ef & 32) ? "ADJOINT_INTEGRATE_1RAY: ray crossed too many cells without leaving the grid"
           : (ef & 16) ? "ADJOINT_INTEGRATE_1RAY: The maximum number of subgrid intervals for calculation "
                         "of the radiance along the ray path has been exceeded."
           : (ef & 1) ? "ADJOINT_INTEGRATE_1RAY: SO<0"

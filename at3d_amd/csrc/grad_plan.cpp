@@ -60,7 +60,7 @@ bool interp_weights(const Plan& p, float X, float Y, float Z, float* wt, int32_t
 
 }  // namespace
 
-int build_grad_plan(const Plan& p, const at3d_deriv_desc& dd, GradPlan& g, std::string& err) {
+int build_grad_plan(const Plan& p, const at3d_deriv_desc& dd, GradPlan& g, bool sun_paths, std::string& err) {
   const at3d_scene_desc& d = p.d;
   const int npg = d.npx * d.npy * d.npz, npts = p.npts, ML = p.ml, nl = p.nleg + 1;
   const bool deltam = d.deltam != 0;
@@ -196,6 +196,7 @@ int build_grad_plan(const Plan& p, const at3d_deriv_desc& dd, GradPlan& g, std::
       }
     }
   }
+  if (!sun_paths) return AT3D_OK;
   // sun paths, transposed to the property grid.  The reference stores each
   // point's path in a column of LONGEST_PATH_PTS slots (the longest path) and
   // COMPUTE_DIRECT_BEAM_DERIV_ADJOINT (shdomsub4.f:4117-4143) reads a column

@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "direct_beam.h"
 #include "medium_point.h"
 #include "shdom_geom.h"
 
@@ -439,9 +440,8 @@ struct GradPointArgs {
   const float* dlegp;          // [numder][maxpg][ml+1]
   const float* dfj;            // [numder][npts][8]
   const float* dalbm;
-  const int32_t* bp_off;       // [maxpg+1] sun paths by property point
-  const int32_t* bp_ip;
-  const float* bp_w;
+  double* sunw;                // [maxpg] sum of sun-path x beam weights (zeroed)
+  int32_t* path_len;           // [npts + 1] cells of each point's sun path; the longest (zeroed)
 };
 
 void launch_dir_source_grad(hipStream_t st, const float* raw, int ldd, int ndir, const float* ext,
@@ -474,6 +474,8 @@ void launch_adjoint_rays(hipStream_t st, const AdjArgs& a);
 // GRAD8 of every source slot in every ray direction, then the Jacobian.
 void launch_jacobian(hipStream_t st, const GradPointArgs& g, const JacArgs& j, float* g8t);
 void launch_grad_points(hipStream_t st, const GradPointArgs& a);
-void launch_grad_beam(hipStream_t st, const GradPointArgs& a);
+// The direct-beam term: the sun paths of every grid point (trace geometry `b`
+// with device pointers), then the property points.
+void launch_grad_beam(hipStream_t st, const GradPointArgs& a, const DirectBeamGeom& b, const float* gridpos, int* err);
 
 }  // namespace at3d

@@ -648,6 +648,7 @@ int state_create(const Plan& p, State& s, std::string& err) {
     TRY(upload(s, d_zl, p.zlevels.data(), p.zlevels.size(), err));
     beam.ext = d_ext;
     beam.zl = d_zl;
+    s.beam = beam;
     launch_direct_beam(s.stream, beam, s.gridpos, p.npts, 1.0f / fabsf(p.d.solarmu), s.dirflux, s.f0, s.errflag);
     HIPCHK(hipGetLastError());
     int ef = 0;

@@ -10,6 +10,7 @@
 #include <vector>
 
 #include "devmem.h"
+#include "direct_beam.h"
 #include "host_plan.h"
 #include "kernels.h"
 
@@ -31,6 +32,7 @@ struct State {
   float splitcrit = 0.0f;       // SPLITCRIT of the last splitting test
   float albmax = 0.0f;          // the largest scattering albedo (a single iteration below SOLACC)
   float* beam_ext = nullptr;    // device medium: the direct beam's property-grid extinction
+  DirectBeamGeom beam;          // the direct beam's trace, device pointers
   std::vector<int32_t> medium_cls_h;   // device medium: source classes and total extinction
   std::vector<float> medium_ext_h;     // of every point (for the ring layout)
   int device = 0;   // HIP device the state was created on
