@@ -258,16 +258,8 @@ int state_levis_gradient(State& s, const at3d_deriv_desc& dd, int64_t nrays, con
     const int rc = direction_tables(s, nrays, mu, phi, t, err);
     if (rc) return rc;
   }
-  const int ndir = t.ndir, ldd = t.ldd, ML = p.ml, np = p.numphase, nsa = p.nscatangle;
+  const int ndir = t.ndir, ldd = t.ldd, ML = p.ml, np = p.numphase;
   const int npts = p.npts, maxpg = g.maxpg, numder = g.numder, npart = p.npart, nl1 = ML + 1;
-  std::vector<float> dssd((size_t)ndir * g.dnumphase, 0.f);
-  for (int d = 0; d < ndir; d++) {
-    const int j = t.sa_j[d];
-    const float f = t.sa_f[d];
-    for (int k = 0; k < g.dnumphase; k++)
-      dssd[(size_t)d * g.dnumphase + k] =
-          (1 - f) * g.dphasetab[(size_t)k * nsa + j - 1] + f * g.dphasetab[(size_t)k * nsa + j];
-  }
   std::vector<float> dlegp((size_t)numder * maxpg * nl1, 0.f);
   for (int idr = 0; idr < numder; idr++) {
     const int ipa = g.partder[idr];
@@ -284,8 +276,6 @@ int state_levis_gradient(State& s, const at3d_deriv_desc& dd, int64_t nrays, con
       }
     }
   }
-  std::vector<float> topval(nrays);
-  for (int64_t i = 0; i < nrays; i++) topval[i] = (mu[i] < 0.0) ? p.d.skyrad : 0.0f;
   std::vector<int32_t> partder(g.partder), doexact(g.doexact);
 
   // ---- device buffers (one block, grown on demand) ----
@@ -297,12 +287,19 @@ int state_levis_gradient(State& s, const at3d_deriv_desc& dd, int64_t nrays, con
     return o;
   };
   const size_t tab = (size_t)s.nptsp * ldd;
-  const size_t o_yd = carve(t.Yd.size() * 4), o_g = carve(t.G.size() * 4), o_ss = carve(t.ssd.size() * 4);
-  const size_t o_dss = carve(dssd.size() * 4);
+  const size_t o_yd = carve((size_t)ldd * s.ld * 4), o_g = carve((size_t)ndir * nl1 * 4);
+  const size_t o_ss = carve((size_t)ndir * np * 4), o_dss = carve((size_t)ndir * g.dnumphase * 4);
+  const size_t o_dirs = carve((size_t)ndir * 16), o_dpt = carve(g.dphasetab.size() * 4);
+  // rays with directions of their own: the source and GRAD8 at the points
+  // around each ray's path alone (the Jacobian takes the full tables)
+  bool pairs = njac == 0 && pair_source_pays(s, nrays, ndir);
+  const int cap = pair_cap(p);
+  const size_t o_cnt = carve(pairs ? (size_t)nrays * 4 : 0), o_over = carve(4);
+  const size_t o_list = carve(pairs ? (size_t)nrays * cap * 4 : 0);
   const size_t o_raw = carve(tab * 4), o_dsrc = carve(tab * 4), o_pre = carve(tab * 4), o_ss8 = carve(tab * 4);
   const size_t o_x = carve(nr * 4), o_y = carve(nr * 4), o_z = carve(nr * 4);
   const size_t o_mu = carve(nr * 8), o_phi = carve(nr * 8), o_dir = carve(nr * 4);
-  const size_t o_top = carve(nr * 4), o_out = carve(nr * 4), o_adj = carve(nr * 8);
+  const size_t o_out = carve(nr * 4), o_adj = carve(nr * 8);
   const size_t o_bsrc = carve(tab * 8), o_erad = carve((size_t)npts * 8), o_bw = carve((size_t)npts * 8);
   const size_t o_grad = carve((size_t)numder * maxpg * 8);
   const size_t o_sjo = carve(sp.sj_off.size() * 4), o_sji = carve(sp.sj_iph.size() * 4);
@@ -344,17 +341,14 @@ int state_levis_gradient(State& s, const at3d_deriv_desc& dd, int64_t nrays, con
     if (bytes == 0) return hipSuccess;
     return hipMemcpyAsync(B + o, src, bytes, hipMemcpyHostToDevice, s.stream);
   };
-  HIPCHK(up(o_yd, t.Yd.data(), t.Yd.size() * 4));
-  HIPCHK(up(o_g, t.G.data(), t.G.size() * 4));
-  HIPCHK(up(o_ss, t.ssd.data(), t.ssd.size() * 4));
-  HIPCHK(up(o_dss, dssd.data(), dssd.size() * 4));
+  HIPCHK(up(o_dirs, t.dirs.data(), (size_t)ndir * 16));
+  HIPCHK(up(o_dpt, g.dphasetab.data(), g.dphasetab.size() * 4));
   HIPCHK(up(o_x, x, nr * 4));
   HIPCHK(up(o_y, y, nr * 4));
   HIPCHK(up(o_z, z, nr * 4));
   HIPCHK(up(o_mu, mu, nr * 8));
   HIPCHK(up(o_phi, phi, nr * 8));
   HIPCHK(up(o_dir, t.dir_of_ray.data(), nr * 4));
-  HIPCHK(up(o_top, topval.data(), nr * 4));
   HIPCHK(up(o_sjo, sp.sj_off.data(), sp.sj_off.size() * 4));
   HIPCHK(up(o_sji, sp.sj_iph.data(), sp.sj_iph.size() * 4));
   HIPCHK(up(o_sjc, sp.sj_coef.data(), sp.sj_coef.size() * 4));
@@ -406,10 +400,17 @@ int state_levis_gradient(State& s, const at3d_deriv_desc& dd, int64_t nrays, con
   float* dsrc = reinterpret_cast<float*>(B + o_dsrc);
   float* srcpre = reinterpret_cast<float*>(B + o_pre);
   float* ss8 = reinterpret_cast<float*>(B + o_ss8);
-  launch_sh_dot(s.stream, s.S, reinterpret_cast<float*>(B + o_yd), raw, s.nptsp, ldd, s.ld, ldd, npts, ndir);
-  launch_dir_source_grad(s.stream, raw, ldd, ndir, s.ext, s.ns, s.lofj, s.tms,
-                         reinterpret_cast<float*>(B + o_g), s.ss_off, s.ss_iph, s.ss_coef,
-                         reinterpret_cast<float*>(B + o_ss), np, ML, npts, 0, dsrc, srcpre, ss8);
+  {
+    DirectionArgs da = direction_args(s, ndir, ldd);
+    da.dirs = reinterpret_cast<double*>(B + o_dirs);
+    da.Yd = reinterpret_cast<float*>(B + o_yd);
+    da.G = reinterpret_cast<float*>(B + o_g);
+    da.ssd = reinterpret_cast<float*>(B + o_ss);
+    da.dphasetab = reinterpret_cast<float*>(B + o_dpt);
+    da.dnumphase = g.dnumphase;
+    da.dssd = reinterpret_cast<float*>(B + o_dss);
+    launch_direction_tables(s.stream, da);
+  }
   const float albpi = p.d.gndalbedo / acosf(-1.0f);
   launch_render_bottom(s.stream, s.fluxes, s.dirflux, s.bcbot, (int)p.bcbot.size(), albpi, s.bcrad_render);
   RayArgs a;
@@ -427,7 +428,6 @@ int state_levis_gradient(State& s, const at3d_deriv_desc& dd, int64_t nrays, con
   a.open_y = (p.bcflag >> 1) & 1;
   a.ext = s.ext;
   a.dsrc = dsrc;
-  a.ldd = ldd;
   a.bot_index = s.bot_index;
   a.bcrad_bot = s.bcrad_render;
   a.camx = reinterpret_cast<float*>(B + o_x);
@@ -436,7 +436,7 @@ int state_levis_gradient(State& s, const at3d_deriv_desc& dd, int64_t nrays, con
   a.cammu = reinterpret_cast<double*>(B + o_mu);
   a.camphi = reinterpret_cast<double*>(B + o_phi);
   a.dir_of_ray = reinterpret_cast<int32_t*>(B + o_dir);
-  a.topval = reinterpret_cast<float*>(B + o_top);
+  a.skyrad = p.d.skyrad;
   a.nrays = (int)nrays;
   a.tautol = p.d.tautol;
   a.transcut = p.d.transcut;
@@ -444,13 +444,47 @@ int state_levis_gradient(State& s, const at3d_deriv_desc& dd, int64_t nrays, con
   a.out = reinterpret_cast<float*>(B + o_out);
   a.errflag = s.errflag;
   (void)hipEventRecord(s.ev[6], s.stream);
-  launch_render(s.stream, a);
-  HIPCHK(hipGetLastError());
+  PairArgs pa = pair_args(s);
+  pa.list = reinterpret_cast<int32_t*>(B + o_list);
+  pa.cnt = reinterpret_cast<int32_t*>(B + o_cnt);
+  pa.over = reinterpret_cast<int*>(B + o_over);
+  pa.cap = cap;
+  pa.Yd = reinterpret_cast<float*>(B + o_yd);
+  pa.G = reinterpret_cast<float*>(B + o_g);
+  pa.ssd = reinterpret_cast<float*>(B + o_ss);
+  pa.dsrc = dsrc;
+  pa.srcpre = srcpre;
+  pa.ss8 = ss8;
+  pa.bsrc = reinterpret_cast<double*>(B + o_bsrc);
   std::vector<float> vis(nr);
   int ef = 0;
-  HIPCHK(hipMemcpyAsync(vis.data(), B + o_out, nr * 4, hipMemcpyDeviceToHost, s.stream));
-  HIPCHK(hipMemcpyAsync(&ef, s.errflag, sizeof(int), hipMemcpyDeviceToHost, s.stream));
-  HIPCHK(hipStreamSynchronize(s.stream));
+  for (;;) {
+    a.ps = pairs ? 1 : ldd;
+    a.ds = pairs ? (size_t)s.nptsp : 1;
+    if (pairs) {
+      HIPCHK(hipMemsetAsync(pa.over, 0, sizeof(int), s.stream));
+      // the adjoint traversal weighs the extinctions of a cell in another
+      // order: its paths may end a rounding later
+      RayArgs m = a;
+      m.transcut = 0.99 * a.transcut;
+      launch_ray_pairs(s.stream, m, pa);
+      launch_pair_source(s.stream, a, pa);
+    } else {
+      launch_sh_dot(s.stream, s.S, reinterpret_cast<float*>(B + o_yd), raw, s.nptsp, ldd, s.ld, ldd, npts, ndir);
+      launch_dir_source_grad(s.stream, raw, ldd, ndir, s.ext, s.ns, s.lofj, s.tms,
+                             reinterpret_cast<float*>(B + o_g), s.ss_off, s.ss_iph, s.ss_coef,
+                             reinterpret_cast<float*>(B + o_ss), np, ML, npts, 0, dsrc, srcpre, ss8);
+    }
+    launch_render(s.stream, a);
+    HIPCHK(hipGetLastError());
+    int over = 0;
+    HIPCHK(hipMemcpyAsync(vis.data(), B + o_out, nr * 4, hipMemcpyDeviceToHost, s.stream));
+    HIPCHK(hipMemcpyAsync(&ef, s.errflag, sizeof(int), hipMemcpyDeviceToHost, s.stream));
+    if (pairs) HIPCHK(hipMemcpyAsync(&over, pa.over, sizeof(int), hipMemcpyDeviceToHost, s.stream));
+    HIPCHK(hipStreamSynchronize(s.stream));
+    if (!over) break;
+    pairs = false;   // a ray crosses more cells than its list holds: every point's source
+  }
   if (ef) {
     err = (ef & 1)   ? "INTEGRATE_1RAY: SO<0"
           : (ef & 2) ? "FIND_BOUNDARY_RADIANCE: Not at boundary"
@@ -491,7 +525,7 @@ int state_levis_gradient(State& s, const at3d_deriv_desc& dd, int64_t nrays, con
   // ---- phase 3: adjoint traversal and contraction ----
   HIPCHK(up(o_adj, adjw_ray.data(), nr * 8));
   if (njac > 0) HIPCHK(up(o_jw, jacw_ray.data(), nr * 8));
-  HIPCHK(hipMemsetAsync(B + o_bsrc, 0, tab * 8, s.stream));
+  if (!pairs) HIPCHK(hipMemsetAsync(B + o_bsrc, 0, tab * 8, s.stream));
   HIPCHK(hipMemsetAsync(B + o_erad, 0, (size_t)npts * 8, s.stream));
   HIPCHK(hipMemsetAsync(B + o_bw, 0, (size_t)npts * 8, s.stream));
   HIPCHK(hipMemsetAsync(B + o_grad, 0, (size_t)numder * maxpg * 8, s.stream));
@@ -522,7 +556,8 @@ int state_levis_gradient(State& s, const at3d_deriv_desc& dd, int64_t nrays, con
   GradPointArgs G;
   G.npts = npts;
   G.ndir = ndir;
-  G.ldd = ldd;
+  G.ps = a.ps;
+  G.ds = a.ds;
   G.ld = s.ld;
   G.ml = ML;
   G.numder = numder;
@@ -570,7 +605,10 @@ int state_levis_gradient(State& s, const at3d_deriv_desc& dd, int64_t nrays, con
   G.dalbm = reinterpret_cast<float*>(B + o_dalbm);
   G.sunw = reinterpret_cast<double*>(B + o_sunw);
   G.path_len = reinterpret_cast<int32_t*>(B + o_len);
-  launch_grad_points(s.stream, G);
+  if (pairs)
+    launch_grad_pairs(s.stream, G, a, pa);
+  else
+    launch_grad_points(s.stream, G);
   if (ess) launch_grad_beam(s.stream, G, s.beam, s.gridpos, s.errflag);
   if (njac > 0) {
     JacArgs J;

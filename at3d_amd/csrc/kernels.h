@@ -324,8 +324,8 @@ struct RayArgs {
   int nx, ny, nz, nx1, ny1, nyc;
   int open_x, open_y;
   const float* ext;        // [npts]
-  const float* dsrc;       // [npts][ldd]
-  int ldd;
+  const float* dsrc;       // direction source of point p, direction d at p * ps + d * ds
+  size_t ps = 0, ds = 1;
   int nst = 1;             // Stokes components: dsrc rows hold nst blocks of `cst`
   int cst = 0;             // directions (I, Q, U); out is [nrays][nst]
   const int32_t* bot_index;  // [npts] bottom boundary index or -1
@@ -336,7 +336,7 @@ struct RayArgs {
   const double* cammu;
   const double* camphi;
   const int32_t* dir_of_ray;
-  const float* topval;       // [nrays] downwelling radiance at the domain top
+  float skyrad;              // downwelling radiance at the domain top
   int nrays;
   double tautol, transcut;
   int nosurface;
@@ -352,6 +352,51 @@ void launch_dir_source_finish(hipStream_t st, const float* raw, int ldd, int ndi
                               const float* ssd, int numphase, int ml, int npts, int single_scatter,
                               int tms_on, float* dsrc);
 void launch_render(hipStream_t st, const RayArgs& a);
+// The tables of `nd` ray directions (dirs: mu, phi each; rows nd .. ldd-1 of Yd
+// are zeroed) from the solar harmonics and the phase table.
+struct DirectionArgs {
+  const double* dirs;      // [nd][2]
+  int nd, ldd, ld, ml, mm, nlm, numphase, nsa;
+  const float* ysun;       // [nlm]
+  const int* lofj;         // [nlm]
+  const float* phasetab;   // [numphase][nsa], null without delta-M
+  float solarmu, solaraz;
+  float* Yd;               // [ldd][ld] spherical harmonics
+  float* G;                // [nd][ml+1] truncated single scatter: sum over m of Y_J(dir) Y_J(sun)
+  float* ssd;              // [nd][numphase] the phase table at the solar scattering angle
+  // the derivative phase table at the same angle (gradient), or null
+  const float* dphasetab = nullptr;   // [dnumphase][nsa]
+  int dnumphase = 0;
+  float* dssd = nullptr;   // [nd][dnumphase]
+};
+void launch_direction_tables(hipStream_t st, const DirectionArgs& a);
+// Where every ray has a direction of its own: the points around the cells each
+// ray crosses (cap per ray, counts in cnt; *over set when one has more), and the
+// direction source of those (point, direction) pairs alone.  a.ps / a.ds place
+// an entry; srcpre, ss8, bsrc (zeroed) for the gradient, else null.
+struct PairArgs {
+  int32_t* list;           // [nrays][cap]
+  int32_t* cnt;            // [nrays]
+  int* over;
+  int cap;
+  const float* S;          // [npts][ld]
+  const float* Yd;         // [ndir][ld]
+  const int* ns;
+  const int* lofj;
+  const float* tms;        // [npts][ml+1]
+  const float* G;
+  const int32_t* ss_off;
+  const int32_t* ss_iph;
+  const float* ss_coef;
+  const float* ssd;
+  int ld, ml, mm, numphase, single_scatter, tms_on;
+  float* dsrc;
+  float* srcpre = nullptr;
+  float* ss8 = nullptr;
+  double* bsrc = nullptr;
+};
+void launch_ray_pairs(hipStream_t st, const RayArgs& a, const PairArgs& p);
+void launch_pair_source(hipStream_t st, const RayArgs& a, const PairArgs& p);
 // The polarized direction source: raw rows [npts][ldd] hold I, Q, U blocks of
 // `cst` columns each; G3 [3][ndir][ml+1] the truncated single-scatter
 // factors of I (element 1) and of Q and U (elements 2 and 6 with the sun's
@@ -379,13 +424,13 @@ void launch_sh_dot_qu(hipStream_t st, const float* S, size_t plane, const float*
 
 struct AdjArgs {
   RayArgs r;                   // geometry, dsrc (source x ext), rays, boundary
-  const float* ss8;            // [npts][ldd] exact single scatter x ext
+  const float* ss8;            // exact single scatter x ext, placed as dsrc
   const double* adj_weight;    // [nrays] adjoint x ray x Stokes weight
   const float* dirflux;        // [npts]
   float opi_gndalbedo;         // ground albedo / pi (FL Lambertian)
   int exact_single_scatter;
   int max_intervals;           // sub-step intervals a ray may record
-  double* bsrc;                // [npts][ldd] source-gradient weights
+  double* bsrc;                // source-gradient weights, placed as dsrc
   double* erad;                // [npts] radiance-term weights
   double* beamw;               // [npts] direct-beam weights
   // Jacobian rows (GRAD_INTEGRATE_1RAY): per ray, the same three weights with
@@ -401,9 +446,10 @@ struct AdjArgs {
 };
 
 struct GradPointArgs {
-  int npts, ndir, ldd, ld, ml, numder, npart, maxpg, numphase, dnumphase;
+  int npts, ndir, ld, ml, numder, npart, maxpg, numphase, dnumphase;
+  size_t ps, ds;               // bsrc and srcpre of point p, direction d at p * ps + d * ds
   float secmu0;
-  const double* bsrc;
+  double* bsrc;
   const double* erad;
   const double* beamw;
   double* grad;                // [numder][maxpg]
@@ -420,7 +466,7 @@ struct GradPointArgs {
   const int32_t* sj_iph;
   const float* sj_coef;
   const float* albedo;         // [npart][npts]
-  const float* srcpre;         // [npts][ldd]
+  const float* srcpre;
   const int8_t* scatj_ok;      // [npart][npts]
   const float* legt_s;         // [npart][npts][ml+1] delta-M scaled mixed phase (npart > 1)
   const float* f_s;            // [npart][npts]
@@ -474,6 +520,8 @@ void launch_adjoint_rays(hipStream_t st, const AdjArgs& a);
 // GRAD8 of every source slot in every ray direction, then the Jacobian.
 void launch_jacobian(hipStream_t st, const GradPointArgs& g, const JacArgs& j, float* g8t);
 void launch_grad_points(hipStream_t st, const GradPointArgs& a);
+// The same over the listed (point, direction) pairs of each ray.
+void launch_grad_pairs(hipStream_t st, const GradPointArgs& a, const RayArgs& r, const PairArgs& p);
 // The direct-beam term: the sun paths of every grid point (trace geometry `b`
 // with device pointers), then the property points.
 void launch_grad_beam(hipStream_t st, const GradPointArgs& a, const DirectBeamGeom& b, const float* gridpos, int* err);

@@ -404,6 +404,7 @@ size_t plan_footprint_bytes(const Plan& p) {
     b += npts * 4 * (1 + 2 * (size_t)p.npw * p.npart) + npts * 4 * (4 + 3 * ml1 + (2 + 2 * (size_t)p.npw) * p.npart) +
          (size_t)p.d.npx * p.d.npy * p.d.npz * 4 * (4 * (size_t)p.npart + 1) + (npts / p.nz) * (size_t)p.nz * 80;
   b += (size_t)p.d.npx * p.d.npy * p.d.npz * 4 + p.zlevels.size() * 4;   // direct-beam extinction
+  b += p.phasetab.size() * 4;
   return b;
 }
 
@@ -710,6 +711,7 @@ int state_create(const Plan& p, State& s, std::string& err) {
     for (int c = s.oct_col_base[o]; c < s.oct_col_base[o] + s.oct_nord[o]; c++) coct[c] = (int8_t)o;
   TRY(upload(s, s.col_oct, coct.data(), coct.size(), err));
   // rendering constants
+  if (p.d.deltam && p.nst == 1) TRY(upload(s, s.phasetab, p.phasetab.data(), p.phasetab.size(), err));
   if (!p.medium_on_device) {
     TRY(upload(s, s.tms, p.tms.data(), p.tms.size(), err));
     TRY(upload(s, s.ss_off, p.ss_off.data(), p.ss_off.size(), err));

@@ -170,14 +170,26 @@ struct DirTables {
   int ndir = 0, ldd = 0;
   std::vector<int32_t> dir_of_ray;                  // [nrays]
   std::vector<std::pair<double, double>> dirs;      // (mu, phi) of each direction
+  // polarized states only (a scalar state's tables are made on the device)
   std::vector<float> Yd, G, ssd;                    // [ldd][ld], [ndir][ml+1], [ndir][numphase]
   // polarized: the Q / U rows [2 ldd][2 ld] (Q of direction d: elements 2 and
   // 5; U at ldd + d: elements 6 and 3), the Q and U truncation factors
   // [2][ndir][ml+1] after G, and the rotated I-Q phase values [ndir][numphase]
   std::vector<float> Yqu, ssq, ssu;
-  std::vector<int32_t> sa_j;                        // scattering-angle table index (1-based lower)
-  std::vector<float> sa_f;                          // and interpolation fraction
 };
+// Offsets of a call's arrays in its device block.
+struct RayCarve {
+  size_t off = 0;
+  size_t take(size_t bytes) {
+    const size_t o = off;
+    off = (off + bytes + 255) / 256 * 256;
+    return o;
+  }
+};
+DirectionArgs direction_args(const State& s, int ndir, int ldd);
+PairArgs pair_args(const State& s);
+int pair_cap(const Plan& p);
+bool pair_source_pays(const State& s, int64_t nrays, int ndir);
 int direction_tables(const State& s, int64_t nrays, const double* mu, const double* phi, DirTables& t,
                      std::string& err);
 
