@@ -390,10 +390,13 @@ int at3d_state_get(at3d_state* st, const char* name, void* dst, size_t nbytes, c
       return AT3D_ERR_DEVICE;
     }
     float* out = static_cast<float*>(dst);
-    const bool level_order = k == "do_source" && s.dosrc_level_order;
+    const int order = k == "do_source" ? s.dosrc_order : 0;
     for (size_t k2 = 0; k2 < nang; k2++) {
       const size_t c = s.col_of_ref[k2];
-      if (level_order) {
+      if (order == 2) {
+        const int32_t* perm = s.plane_perm_h.data() + (size_t)(s.plane_type_h[c] & 3) * s.nptsp;
+        for (size_t q = 0; q < npts; q++) out[k2 * npts + perm[q]] = tmp[c * s.nptsp + q];
+      } else if (order == 1) {
         int o = 0;
         while (o < 7 && (int)c >= s.oct_col_base[o] + s.oct_nord[o]) o++;
         const int32_t* pos = s.oct_pos_h.data() + (size_t)o * npts;
@@ -620,6 +623,12 @@ int at3d_state_set_option(at3d_state* st, const char* key, int32_t value, char* 
   }
   if (k == "sweep_ring") {
     st->s.use_ring = value < 0 ? 0 : (value > 2 ? 2 : value);
+    if (st->s.use_ring == 2) {
+      std::string e;
+      const int rc = ensure_ring(st->s, e);
+      if (rc) set_err(err, errlen, e.c_str());
+      return rc;
+    }
     return AT3D_OK;
   }
   if (k == "render_correct_interpolate") {
@@ -659,11 +668,14 @@ double at3d_state_timing(const at3d_state* st, const char* key) {
   if (k == "sweep_launches") return s.nsweep_launch;
   if (k == "sweep_kernel") return s.tsum[6];
   if (k == "device_bytes") return (double)s.device_bytes;
-  if (k == "sweep_ring")
-    return (s.ring_ok && s.use_ring && !s.force_general && (s.use_ring == 2 || !s.ring_chain)) ? 1.0 : 0.0;
-  if (k == "sweep_ring_lds") return (double)(s.ring_full ? s.ring_lds_full : s.ring_lds);
+  // a level-ordered sweep (by planes or the ring)
+  if (k == "sweep_ring") return planes_active(s) || ring_active(s) ? 1.0 : 0.0;
+  if (k == "sweep_planes") return planes_active(s) ? 1.0 : 0.0;
+  if (k == "sweep_ring_lds")
+    return (double)(planes_active(s) ? s.plane_lds : s.ring_full ? s.ring_lds_full : s.ring_lds);
   if (k == "sweep_ring_slots") return s.slots;
-  if (k == "sweep_ring4") return s.ring4;
+  // the grid's ring holds radiances alone, whichever sweep runs
+  if (k == "sweep_ring4") return s.ring_tried ? s.ring4 : ring_wants_radiances_alone(s);
   if (k == "sweep_ring_full") return s.ring_full;
   if (k == "sweep_sectors") return s.nsectors;
   if (k == "sweep_general_points") return s.ngeneral;

@@ -40,10 +40,11 @@ void launch_sh_to_do(hipStream_t st, const float* S, const float* Yc, const floa
                      const int* stop = nullptr);
 // Level-ordered variant: dosrc[c][q] = max(0, sum_J S[perm_o[q]][J] * Yc[c][J]) * ext[perm_o[q]]
 // for each column c of octant o, perm_o = oct_perm + o * mp (the octant's
-// positions: its levels, boundary points included).  tiles[t] = {octant,
-// first column, columns (<= 48), 0}.  S[p][J] must be zero for J >= ns[p].
+// positions: its levels, boundary points included).  tiles[t] = {order, first
+// entry of `cols`, columns (<= 48), offset added to a column}; cols null: the
+// columns themselves.  S[p][J] must be zero for J >= ns[p].
 void launch_sh_to_do_perm(hipStream_t st, const float* S, const float* Yc, const float* ext,
-                          const int* ns, const int32_t* oct_perm, const int4* tiles, int ntiles,
+                          const int* ns, const int32_t* oct_perm, const int4* tiles, const int32_t* cols, int ntiles,
                           float* dosrc, int mp, int ld, int ldp, int npts, const int* stop = nullptr);
 // The polarized Q and U rows of the point-ordered SH->DO (no clamp): S the
 // Q plane, the U plane `plane` floats on; Yc [ncp][2 ld] with ncp = 2 ldo
@@ -55,8 +56,9 @@ void launch_sh_to_do_qu(hipStream_t st, const float* S, size_t plane, const floa
 // 2 ld long (the Q-plane terms then the U-plane terms), one row per output
 // column of a Q / U tile; no clamp at zero.
 void launch_sh_to_do_perm_qu(hipStream_t st, const float* S, size_t plane, const float* Yc, const float* ext,
-                             const int* ns, const int32_t* oct_perm, const int4* tiles, int ntiles,
-                             float* dosrc, int mp, int ld, int ldp, int npts, const int* stop = nullptr);
+                             const int* ns, const int32_t* oct_perm, const int4* tiles, const int32_t* cols,
+                             int ntiles, float* dosrc, int mp, int ld, int ldp, int npts,
+                             const int* stop = nullptr);
 // R[p][J] = (J < nr[p]) ? sum_c dorad[c][p] * Wc[c][J] : 0
 // dorad [ldo][ldp] (rows beyond nang zero), Wc [ldo][ld] (rows beyond nang zero), R [mp][ld].
 void launch_do_to_sh(hipStream_t st, const float* dorad, const float* Wc, const int* nr, float* R,
@@ -186,6 +188,31 @@ void launch_sweep_ring(hipStream_t st, const SweepArgs& a, int col0, int ncol, s
 void launch_sweep_preset(hipStream_t st, const SweepArgs& a, bool up, int col0, int ncol);
 // One workgroup per ordinate column col0 .. col0+ncol-1, all levels of its octant.
 void launch_sweep_columns(hipStream_t st, const SweepArgs& a, int col0, int ncol);
+// ---- sweep_planes.hip: plane-ordered sweep of open base grids -------------
+// Per axis t (0: z, 1: x, 2: y) the planes across it, in ascending coordinate:
+// within plane k a point's natural index is s = y + ny x (z), z + nz y (x) or
+// z + nz x (y); the source rows of an axis's columns hold plane k at k * M ..
+// (k + 1) * M (M points a plane), within a plane in the order of pidx.
+struct PlaneArgs {
+  const int8_t* col_type = nullptr;   // [ncols] axis; + 4: an open side's plane is swept by the other
+                                      // horizontal axis, not by z
+  const uint16_t* pidx = nullptr;     // [3][npts] natural index of each position of a source row
+  const float* ext = nullptr;         // [3][npts] extinction, plane by plane, natural order
+  double dx = 0, dy = 0;              // horizontal spacings
+};
+// Largest plane: four points a thread of 1024.  With more a thread's registers
+// spill, and the ring is as fast or faster (96 x 96 x 48, ten points a thread:
+// 1012 us a hemisphere against the ring's 984; 128 x 128 x 64 polarized, 16:
+// 16.8 against 5.8 ms).  LDS bytes for planes of mz points across z and ms
+// across x or y.
+constexpr int PLANE_POINTS_MAX = 4096;
+inline size_t plane_lds_bytes(int mz, int ms, int nz) { return ((size_t)(mz > ms ? mz : ms) + nz) * 16; }
+int sweep_planes_max_lds(int mz, int ms, size_t lds);
+void launch_plane_ext(hipStream_t st, const float* ext, float* out, int nx, int ny, int nz);
+// Columns col0 .. col0+ncol-1 with their boundary radiances (a.qu_only_from as
+// for the ring).
+void launch_sweep_planes(hipStream_t st, const SweepArgs& a, const PlaneArgs& p, int col0, int ncol, int mz, int ms,
+                         size_t lds);
 // ---- sweep_chain.hip: point-ordered sweep from per-ordinate records ------
 // Arrays of one state, rows of npts entries per column: in the octant's list
 // order (q while the levels are made), then in the ordinate's level order.

@@ -171,12 +171,53 @@ static SweepArgs sweep_args(const State& s) {
 // points swept just before): there the point-ordered sweep, whose levels are
 // each ordinate's own, is faster (16^3 periodic, NMU 8: 0.7 against 45 ms per
 // iteration).
-static bool ring_active(const State& s) {
+bool ring_active(const State& s) {
+  if (planes_active(s)) return false;
   return s.ring_ok && s.use_ring && !s.force_general && (s.use_ring == 2 || !s.ring_chain);
 }
 
+// The plane-ordered sweep where the grid takes it, unless the ring is asked for.
+bool planes_active(const State& s) { return s.planes_ok && s.use_ring == 1 && !s.force_general; }
+
 // The point-ordered sweep from per-ordinate records (ensure_sweep made them).
-static bool chain_active(const State& s) { return !ring_active(s) && !s.force_general && s.chain == 1; }
+static bool chain_active(const State& s) {
+  return !planes_active(s) && !ring_active(s) && !s.force_general && s.chain == 1;
+}
+
+// Rank and level of every octant's points (the ring's records and the
+// multi-cell traces read them), uploaded on their first use.
+static int ensure_ranks(State& s, std::string& err) {
+  if (s.rank) return AT3D_OK;
+  const Plan& p = *s.plan;
+  TRY(alloc_only(s, s.rank, (size_t)8 * p.npts, err));
+  TRY(alloc_only(s, s.level, (size_t)8 * p.npts, err));
+  for (int o = 0; o < 8; o++) {
+    HIPCHK(hipMemcpyAsync(s.rank + (size_t)o * p.npts, p.oct[o].rank.data(), (size_t)p.npts * 4,
+                          hipMemcpyHostToDevice, s.stream));
+    HIPCHK(hipMemcpyAsync(s.level + (size_t)o * p.npts, p.oct[o].level.data(), (size_t)p.npts * 4,
+                          hipMemcpyHostToDevice, s.stream));
+  }
+  HIPCHK(hipStreamSynchronize(s.stream));
+  return AT3D_OK;
+}
+
+// Whether the ring of this state's grid holds radiances alone: pairs of
+// radiance and source over the five levels that four-point sectors need do
+// not fit in LDS (build_ring_plan, without the layout).
+bool ring_wants_radiances_alone(const State& s) {
+  const Plan& p = *s.plan;
+  if (!p.treeptr.empty()) return false;
+  int slots = 0, nlev = 0;
+  for (int o = 0; o < 8; o++) {
+    if (s.oct_nord[o] <= 0) continue;
+    const std::vector<int32_t>& off = p.oct[o].ring_off;
+    const int n = p.oct[o].ring_nlev;
+    nlev = std::max(nlev, n);
+    for (int L = 0; L <= n && L < (int)off.size(); L++)
+      slots = std::max(slots, off[std::min(n, L + 5)] - off[L]);
+  }
+  return s.force_ring4 || ring_lds_bytes(slots, nlev + 2, 0, 8) > GFX950_LDS_BYTES;
+}
 
 // The level-ordered sweep: each octant's ring order (its levels, with the
 // hemisphere's boundary points as entries of their own), the SH->DO column
@@ -185,6 +226,8 @@ static bool chain_active(const State& s) { return !ring_active(s) && !s.force_ge
 // in LDS or the records do not fit in memory.
 static int setup_ring(const Plan& p, State& s, std::string& err) {
   s.ring_ok = false;
+  s.ring_tried = true;
+  TRY(ensure_ranks(s, err));
   // the step classes and ring layout assume the base grid's regular cells
   if (!p.treeptr.empty()) return AT3D_OK;
   bool used[8];
@@ -204,7 +247,6 @@ static int setup_ring(const Plan& p, State& s, std::string& err) {
     if (!build_ring_plan(p, used, (size_t)maxlds, rp, err, cls, 4)) return AT3D_ERR_NUMERIC;
   }
   const float* total_ext = p.medium_on_device ? s.medium_ext_h.data() : p.total_ext.data();
-  s.ring_chain = false;
   for (int o = 0; o < 8; o++)
     if (used[o] && rp.oct[o].nlev > 0 && (double)p.npts / rp.oct[o].nlev < 4.0) s.ring_chain = true;
   s.sector_points = rp.sector_points;
@@ -373,6 +415,133 @@ static int setup_ring(const Plan& p, State& s, std::string& err) {
 }
 
 
+int ensure_ring(State& s, std::string& err) { return s.ring_tried ? AT3D_OK : setup_ring(*s.plan, s, err); }
+
+// The axis of every ordinate of a plan (device column order is the caller's):
+// the one whose spacing over direction cosine is the shortest, for every layer;
+// + 4 where an open side's own plane is swept by the other horizontal axis.
+// False where the plane-ordered sweep does not apply: periodic or refined
+// grids, ordinates whose axis (or an open side's) changes from layer to layer,
+// planes beyond PLANE_POINTS_MAX.  Steps of equal length (a shared edge) may go
+// by either face.
+static bool plane_types(const Plan& p, std::vector<int8_t>& type, int& mz, int& ms) {
+  if (!p.treeptr.empty() || (p.bcflag & 3) != 3 || p.ipflag != 0) return false;
+  if (p.nx1 < 2 || p.ny1 < 2 || p.nz < 2) return false;
+  const double dx = ((double)p.xgrid[p.nx1 - 1] - p.xgrid[0]) / (p.nx1 - 1);
+  const double dy = ((double)p.ygrid[p.ny1 - 1] - p.ygrid[0]) / (p.ny1 - 1);
+  double zmin = 1e300, zmax = 0.0;
+  for (int k = 0; k + 1 < p.nz; k++) {
+    const double dz = (double)p.zgrid[k + 1] - p.zgrid[k];
+    zmin = std::min(zmin, dz);
+    zmax = std::max(zmax, dz);
+  }
+  if (!(zmin > 0.0) || !(dx > 0.0) || !(dy > 0.0)) return false;
+  // (equal to the rounding of the grid's coordinates)
+  const double eps = 1e-5;
+  type.assign(p.nang, 0);
+  mz = ms = 0;
+  for (int k = 0; k < p.nang; k++) {
+    const OrdGeom& g = p.ords[k].g;
+    const double hx = dx * fabs(g.cxinv), hy = dy * fabs(g.cyinv);
+    const double z0 = zmin * fabs(g.czinv), z1 = zmax * fabs(g.czinv);
+    const double hb = std::min(hx, hy);
+    if (z1 <= hb * (1 + eps)) {
+      type[k] = 0;
+      mz = p.nx1 * p.ny1;
+      continue;
+    }
+    if (hb > z0 * (1 + eps)) return false;   // z in some layers only
+    type[k] = hx <= hy ? 1 : 2;
+    ms = std::max(ms, p.nz * (hx <= hy ? p.ny1 : p.nx1));
+    const double ho = std::max(hx, hy);   // the other horizontal axis, in the side's own plane
+    if (z1 <= ho * (1 + eps)) continue;
+    if (ho > z0 * (1 + eps)) return false;
+    type[k] |= 4;
+  }
+  return std::max(mz, ms) <= PLANE_POINTS_MAX && plane_lds_bytes(mz, ms, p.nz) <= (size_t)GFX950_LDS_BYTES;
+}
+
+// The plane-ordered sweep's orders: per axis the points plane by plane, within
+// a plane grouped by source class (ascending on even planes, descending on odd
+// ones, so classes meet across planes too), and the SH->DO tiles of its columns.
+static int setup_planes(const Plan& p, State& s, std::string& err) {
+  std::vector<int8_t> type;
+  if (!plane_types(p, type, s.plane_mz, s.plane_ms)) return AT3D_OK;
+  s.plane_lds = plane_lds_bytes(s.plane_mz, s.plane_ms, p.nz);
+  if (sweep_planes_max_lds(s.plane_mz, s.plane_ms, s.plane_lds) != 0) {
+    (void)hipGetLastError();
+    return AT3D_OK;
+  }
+  const int nx = p.nx1, ny = p.ny1, nz = p.nz;
+  const size_t np = p.npts;
+  std::vector<int32_t> own;
+  if (!p.medium_on_device) plan_source_class(p, own);
+  const std::vector<int32_t>& cls = p.medium_on_device ? s.medium_cls_h : own;
+  s.plane_perm_h.assign((size_t)3 * s.nptsp, 0);
+  std::vector<uint16_t> pidx(3 * np, 0);
+  const int nk[3] = {nz, nx, ny}, m[3] = {nx * ny, ny * nz, nx * nz};
+  const int nplanes = nz + nx + ny;
+  parallel_for(nplanes, [&](int j) {
+    const int t = j < nz ? 0 : (j < nz + nx ? 1 : 2), k = j - (t == 0 ? 0 : (t == 1 ? nz : nz + nx)), M = m[t];
+    auto point = [&](int q) {
+      if (t == 0) return k + nz * q;                              // q = y + ny x
+      if (t == 1) return q + nz * ny * k;                         // q = z + nz y
+      const int x = q / nz;
+      return q - x * nz + nz * (k + ny * x);                      // q = z + nz x
+    };
+    std::vector<int> start(p.ml + 3, 0);
+    auto bin = [&](int q) { return (k & 1) ? p.ml - cls[point(q)] : cls[point(q)]; };
+    for (int q = 0; q < M; q++) start[bin(q) + 1]++;
+    for (int l = 0; l <= p.ml; l++) start[l + 1] += start[l];
+    int32_t* perm = s.plane_perm_h.data() + (size_t)t * s.nptsp + (size_t)k * M;
+    uint16_t* ix = pidx.data() + (size_t)t * np + (size_t)k * M;
+    for (int q = 0; q < M; q++) {
+      const int at = start[bin(q)]++;
+      perm[at] = point(q);
+      ix[at] = (uint16_t)q;
+    }
+  });
+  for (int t = 0; t < 3; t++)
+    for (int q = p.npts; q < s.nptsp; q++) s.plane_perm_h[(size_t)t * s.nptsp + q] = q;
+  // device columns and the tiles of each axis
+  s.plane_type_h.assign(s.ldo, 0);
+  std::vector<int32_t> cols;
+  std::vector<int4> tiles;
+  for (int k = 0; k < p.nang; k++) s.plane_type_h[s.col_of_ref[k]] = type[k];
+  for (int t = 0; t < 3; t++) {
+    const int first = (int)cols.size();
+    for (int c = 0; c < p.nang; c++)
+      if ((s.plane_type_h[c] & 3) == t) cols.push_back(c);
+    for (int c = first; c < (int)cols.size(); c += 48)
+      tiles.push_back(make_int4(t, c, std::min(48, (int)cols.size() - c), 0));
+  }
+  uint16_t* d_pidx = nullptr;
+  float* d_ext = nullptr;
+  int8_t* d_type = nullptr;
+  TRY(upload(s, s.plane_perm, s.plane_perm_h.data(), s.plane_perm_h.size(), err));
+  TRY(upload(s, d_pidx, pidx.data(), pidx.size(), err));
+  TRY(upload(s, s.plane_cols, cols.data(), cols.size(), err));
+  TRY(upload(s, s.plane_tiles, tiles.data(), tiles.size(), err));
+  if (s.nst == 3) {
+    // the Q and U rows of each tile's columns: U ldo rows on
+    std::vector<int4> qu(tiles);
+    for (const int4& t : tiles) qu.push_back(make_int4(t.x, t.y, t.z, s.ldo));
+    TRY(upload(s, s.plane_tiles_qu, qu.data(), qu.size(), err));
+  }
+  TRY(upload(s, d_type, s.plane_type_h.data(), s.plane_type_h.size(), err));
+  TRY(alloc_only(s, d_ext, 3 * np, err));
+  launch_plane_ext(s.stream, s.ext, d_ext, nx, ny, nz);
+  HIPCHK(hipGetLastError());
+  s.n_plane_tiles = (int)tiles.size();
+  s.planes.col_type = d_type;
+  s.planes.pidx = d_pidx;
+  s.planes.ext = d_ext;
+  s.planes.dx = ((double)p.xgrid[nx - 1] - p.xgrid[0]) / (nx - 1);
+  s.planes.dy = ((double)p.ygrid[ny - 1] - p.ygrid[0]) / (ny - 1);
+  s.planes_ok = true;
+  return AT3D_OK;
+}
+
 // Device bytes a state of this plan allocates (its arrays and the sweep
 // records; not the per-call render and gradient buffers), for admission by
 // memory footprint before anything is allocated.
@@ -390,14 +559,21 @@ size_t plan_footprint_bytes(const Plan& p) {
   b += 3 * npts * ml1 * 4;               // chi, tc, tms
   b += npts * 4 * 12;                    // per-point scalars, counts, fluxes, partials
   b += npts * 12 + ncells * 57;          // grid positions, cell topology and flags
-  b += 8 * npts * 4 * 4 + npts;          // sweep order: rank, level, level lists, preset
-  b += nang * npts * 16;                 // sweep records
-  b += nang * (size_t)p.nz * 4 * 16 + 8 * nptsp * 4 + 8 * (size_t)p.nz * 4 * 8;  // step classes, ring-order extinction
+  b += npts;                             // boundary points
+  std::vector<int8_t> types;
+  int mz = 0, ms = 0;
+  const bool planes = plane_types(p, types, mz, ms);
+  if (planes) b += 3 * nptsp * 4 + 3 * npts * (2 + 4);   // plane orders and extinctions
   bool chain = !p.treeptr.empty();
   for (int o = 0; o < 8; o++) chain = chain || (p.oct[o].ring_nlev > 0 && (double)npts / p.oct[o].ring_nlev < 4.0);
   if (chain && npts <= 40960)            // point-ordered sweep from records, with its level lists
-    b += nang * npts * chain_point_bytes(p.nst) + nang * 8 + 8 * npts * 4 * 2;
-  b += 8 * nptsp * 4 + 8 * npts * (4 * 4 + 2) + 8 * (npts / 4 + 8) * 20;  // ring layout, face masks, sectors
+    b += nang * npts * chain_point_bytes(p.nst) + nang * 8;
+  if (!planes) b += 8 * npts * 4 * 4;    // sweep order: rank, level, level lists
+  if (!planes && !chain) {
+    b += nang * npts * 16;                 // sweep records
+    b += nang * (size_t)p.nz * 4 * 16 + 8 * nptsp * 4 + 8 * (size_t)p.nz * 4 * 8;  // step classes, ring-order extinction
+    b += 8 * nptsp * 4 + 8 * npts * (4 * 4 + 2) + 8 * (npts / 4 + 8) * 20;  // ring layout, face masks, sectors
+  }
   if (p.host_medium)
     b += p.ss_off.size() * 4 + p.ss_iph.size() * 4 + p.ss_coef.size() * 4;
   else   // the device set-up: at most 8 pairs per species and point, its work arrays
@@ -685,26 +861,17 @@ int state_create(const Plan& p, State& s, std::string& err) {
   for (int i : p.bctop) preset[i] |= 1;
   for (int i : p.bcbot) preset[i] |= 2;
   TRY(upload(s, s.preset, preset.data(), preset.size(), err));
-  // rank and level of every octant (the records and the multi-cell traces
-  // read them); the point-ordered sweep's level lists wait for its first use
-  TRY(alloc_only(s, s.rank, (size_t)8 * p.npts, err));
-  TRY(alloc_only(s, s.level, (size_t)8 * p.npts, err));
   s.nlevels_max = 0;
   {
     int base = 0, lob = 0;
     for (int o = 0; o < 8; o++) {
       const OctantPlan& op = p.oct[o];
-      HIPCHK(hipMemcpyAsync(s.rank + (size_t)o * p.npts, op.rank.data(), (size_t)p.npts * 4,
-                            hipMemcpyHostToDevice, s.stream));
-      HIPCHK(hipMemcpyAsync(s.level + (size_t)o * p.npts, op.level.data(), (size_t)p.npts * 4,
-                            hipMemcpyHostToDevice, s.stream));
       s.oct_pts_base_h[o] = base;
       s.lo_base_h[o] = lob;
       base += (int)op.lvl_pts.size();
       lob += op.nlevels + 1;
       if (s.oct_nord[o] > 0) s.nlevels_max = std::max(s.nlevels_max, op.nlevels);
     }
-    HIPCHK(hipStreamSynchronize(s.stream));
   }
   std::vector<int8_t> coct(s.ldo, 0);
   for (int o = 0; o < 8; o++)
@@ -739,7 +906,12 @@ int state_create(const Plan& p, State& s, std::string& err) {
   }
   TRY(alloc0(s, s.ctl, 1, err));
   s.nr_buf0 = s.nr;
-  TRY(setup_ring(p, s, err));
+  // the level-ordered ring only where neither the planes nor (periodic and
+  // refined grids) the point-ordered sweep is taken
+  for (int o = 0; o < 8; o++)
+    if (s.oct_nord[o] > 0 && p.oct[o].ring_nlev > 0 && (double)p.npts / p.oct[o].ring_nlev < 4.0) s.ring_chain = true;
+  TRY(setup_planes(p, s, err));
+  if (!s.planes_ok && !s.ring_chain && p.treeptr.empty()) TRY(ensure_ring(s, err));
   for (int e = 0; e < State::NEV; e++) HIPCHK(hipEventCreate(&s.ev[e]));
   for (int e = 0; e < 4; e++) HIPCHK(hipEventCreate(&s.ev_sweep[e]));
   for (int e = 0; e < 2; e++) HIPCHK(hipEventCreate(&s.ev_ray[e]));
@@ -820,6 +992,7 @@ static int state_replace(State& s, std::shared_ptr<Plan> owned, SplitFields* f, 
   n.use_graph = s.use_graph;
   n.use_iter_graph = s.use_iter_graph;
   int rc = state_create(q, n, err);
+  if (!rc && n.use_ring == 2) rc = ensure_ring(n, err);
   if (rc) {
     state_free(n);
     return rc;
@@ -1013,7 +1186,7 @@ static void enqueue_sweeps(State& s, const int* stop = nullptr) {
   SweepArgs a = sweep_args(s);
   a.stop = stop;
   const float albpi = p.d.gndalbedo / acosf(-1.0f);
-  const bool ring = ring_active(s), chain = chain_active(s);
+  const bool ring = ring_active(s), chain = chain_active(s), planes = planes_active(s);
   // the ring sweep writes the boundary radiances itself; events around its
   // launches time the sweep kernel alone
   // which ring instantiations each hemisphere's columns need
@@ -1030,7 +1203,7 @@ static void enqueue_sweeps(State& s, const int* stop = nullptr) {
   // surface (Q and U see a zero boundary), so the first launch also runs the
   // upwelling Q and U columns: 5 of the 6 (hemisphere, component) sweeps in
   // one grid, which fills the CUs better than two grids of three
-  const bool merge_qu = ring && s.nst == 3;
+  const bool merge_qu = (ring || planes) && s.nst == 3;
   if (ring) {
     // the first launch is timed from the event the caller records just
     // before this function, the second to the one just after it
@@ -1043,6 +1216,11 @@ static void enqueue_sweeps(State& s, const int* stop = nullptr) {
       needs(0, s.ndown, fast, full);
       launch_sweep_ring(s.stream, a, 0, s.ndown, s.ring_lds, s.ring_lds_full, fast, full);
     }
+    (void)hipEventRecord(s.ev_sweep[1], s.stream);
+  } else if (planes) {
+    SweepArgs a1 = a;
+    if (merge_qu) a1.qu_only_from = s.ndown;
+    launch_sweep_planes(s.stream, a1, s.planes, 0, merge_qu ? p.nang : s.ndown, s.plane_mz, s.plane_ms, s.plane_lds);
     (void)hipEventRecord(s.ev_sweep[1], s.stream);
   } else if (chain) {
     launch_sweep_chain(s.stream, a, s.chain_arrays, 0, s.ndown);
@@ -1059,6 +1237,11 @@ static void enqueue_sweeps(State& s, const int* stop = nullptr) {
     SweepArgs a2 = a;
     if (merge_qu) a2.nst = 1;   // the upwelling I columns alone
     launch_sweep_ring(s.stream, a2, s.ndown, p.nang - s.ndown, s.ring_lds, s.ring_lds_full, fast, full);
+  } else if (planes) {
+    (void)hipEventRecord(s.ev_sweep[2], s.stream);
+    SweepArgs a2 = a;
+    if (merge_qu) a2.nst = 1;
+    launch_sweep_planes(s.stream, a2, s.planes, s.ndown, p.nang - s.ndown, s.plane_mz, s.plane_ms, s.plane_lds);
   } else if (chain) {
     launch_sweep_chain(s.stream, a, s.chain_arrays, s.ndown, p.nang - s.ndown);
   } else {
@@ -1070,6 +1253,7 @@ static void enqueue_sweeps(State& s, const int* stop = nullptr) {
 // The point-ordered sweep's level lists (every octant's non-preset points
 // by level, their start cells and the level offsets), uploaded on its first use.
 static int ensure_point_order(State& s, std::string& err) {
+  TRY(ensure_ranks(s, err));
   if (s.lvl_pts) return AT3D_OK;
   const Plan& p = *s.plan;
   std::vector<int32_t> lp, lc, lo;
@@ -1090,6 +1274,8 @@ static int ensure_point_order(State& s, std::string& err) {
 // sweep's level lists and, where an ordinate's radiances fit in LDS (npts <=
 // 40960) and the records in memory, its per-ordinate records.
 static int ensure_sweep(State& s, std::string& err) {
+  if (planes_active(s)) return AT3D_OK;
+  if (s.use_ring && !s.force_general && (s.use_ring == 2 || !s.ring_chain)) TRY(ensure_ring(s, err));
   if (ring_active(s)) return AT3D_OK;
   TRY(ensure_point_order(s, err));
   if (s.chain || s.force_general) return AT3D_OK;
@@ -1134,7 +1320,7 @@ static int run_sweeps(State& s, std::string& err) {
   // the level-ordered sweep is three launches per pass (and is timed by
   // events between them), the one from records five; k_sweep_columns is
   // replayed from a graph
-  if (!s.use_graph || ring_active(s) || chain_active(s)) {
+  if (!s.use_graph || planes_active(s) || ring_active(s) || chain_active(s)) {
     enqueue_sweeps(s);
     HIPCHK(hipGetLastError());
     return AT3D_OK;
@@ -1190,12 +1376,30 @@ static void accel_solcrit(bool doaccel, float deljdot, float deljold, float delj
 static void enqueue_sh_to_do_qu(State& s, const int* stop) {
   if (s.nst != 3) return;
   const Plan& p = *s.plan;
-  if (ring_active(s))
-    launch_sh_to_do_perm_qu(s.stream, s.S + s.psh, s.psh, s.Yqu, s.ext, s.ns, s.oct_perm, s.sh_tiles_qu,
+  if (planes_active(s))
+    launch_sh_to_do_perm_qu(s.stream, s.S + s.psh, s.psh, s.Yqu, s.ext, s.ns, s.plane_perm, s.plane_tiles_qu,
+                            s.plane_cols, 2 * s.n_plane_tiles, s.dosrc + s.pdo, s.nptsp, s.ld, s.nptsp, p.npts, stop);
+  else if (ring_active(s))
+    launch_sh_to_do_perm_qu(s.stream, s.S + s.psh, s.psh, s.Yqu, s.ext, s.ns, s.oct_perm, s.sh_tiles_qu, nullptr,
                             2 * s.n_sh_tiles, s.dosrc + s.pdo, s.nptsp, s.ld, s.nptsp, p.npts, stop);
   else
     launch_sh_to_do_qu(s.stream, s.S + s.psh, s.psh, s.Yqu, s.ext, s.dosrc + s.pdo, s.nptsp, 2 * s.ldo, s.ld,
                        s.nptsp, p.npts, stop);
+}
+
+// SH->DO of the I rows, in the layout the active sweep reads, then Q and U.
+static void enqueue_sh_to_do(State& s, const int* stop) {
+  const Plan& p = *s.plan;
+  s.dosrc_order = planes_active(s) ? 2 : (ring_active(s) ? 1 : 0);
+  if (s.dosrc_order == 2)
+    launch_sh_to_do_perm(s.stream, s.S, s.Y, s.ext, s.ns, s.plane_perm, s.plane_tiles, s.plane_cols, s.n_plane_tiles,
+                         s.dosrc, s.nptsp, s.ld, s.nptsp, p.npts, stop);
+  else if (s.dosrc_order == 1)
+    launch_sh_to_do_perm(s.stream, s.S, s.Y, s.ext, s.ns, s.oct_perm, s.sh_tiles, nullptr, s.n_sh_tiles, s.dosrc,
+                         s.nptsp, s.ld, s.nptsp, p.npts, stop);
+  else
+    launch_sh_to_do(s.stream, s.S, s.Y, s.ext, s.dosrc, s.nptsp, s.ldo, s.ld, s.nptsp, p.npts, p.nang, stop);
+  enqueue_sh_to_do_qu(s, stop);
 }
 
 static void enqueue_do_to_sh_qu(State& s, const int* stop) {
@@ -1216,12 +1420,7 @@ static void enqueue_iteration(State& s) {
   const Plan& p = *s.plan;
   const int* stop = &s.ctl->stop;
   launch_iter_begin(s.stream, s.ctl);
-  if (ring_active(s))
-    launch_sh_to_do_perm(s.stream, s.S, s.Y, s.ext, s.ns, s.oct_perm, s.sh_tiles, s.n_sh_tiles, s.dosrc,
-                         s.nptsp, s.ld, s.nptsp, p.npts, stop);
-  else
-    launch_sh_to_do(s.stream, s.S, s.Y, s.ext, s.dosrc, s.nptsp, s.ldo, s.ld, s.nptsp, p.npts, p.nang, stop);
-  enqueue_sh_to_do_qu(s, stop);
+  enqueue_sh_to_do(s, stop);
   enqueue_sweeps(s, stop);
   launch_do_to_sh(s.stream, s.dorad, s.W, s.nr, s.R, s.nptsp, s.ld, s.ldo, s.nptsp, p.npts, stop);
   enqueue_do_to_sh_qu(s, stop);
@@ -1235,7 +1434,8 @@ static void enqueue_iteration(State& s) {
 
 // The sweep configuration a captured graph holds.
 static int iteration_key(const State& s) {
-  return (ring_active(s) ? 1 : 0) | (s.force_general ? 2 : 0) | (s.ring_full ? 4 : 0) | (chain_active(s) ? 8 : 0);
+  return (ring_active(s) ? 1 : 0) | (s.force_general ? 2 : 0) | (s.ring_full ? 4 : 0) | (chain_active(s) ? 8 : 0) |
+         (planes_active(s) ? 16 : 0);
 }
 
 // The graph of ITER_BATCH iterations for the NR buffer parity k (0: s.nr is
@@ -1279,7 +1479,6 @@ static int state_solve_graph(State& s, int maxiter, std::string& err) {
   c.solacc = p.d.solacc;
   HIPCHK(hipMemcpyAsync(s.ctl, &c, sizeof c, hipMemcpyHostToDevice, s.stream));
   const int parity = s.nr == s.nr_buf0 ? 0 : 1;
-  s.dosrc_level_order = ring_active(s);
   const int key = iteration_key(s);
   if (!s.iter_exec[parity] || s.iter_key[parity] != key) TRY(capture_iterations(s, parity, err));
   // every batch runs ITER_BATCH iterations unless the device stops: the
@@ -1334,14 +1533,8 @@ static int host_iteration(State& s, bool& fixsh, float& a, int verbose, std::str
   // (into nr_next): it becomes the current NR
   std::swap(s.nr, s.nr_next);
   (void)hipEventRecord(s.ev[0], s.stream);
-  s.dosrc_level_order = ring_active(s);
-  if (s.dosrc_level_order)
-    launch_sh_to_do_perm(s.stream, s.S, s.Y, s.ext, s.ns, s.oct_perm, s.sh_tiles, s.n_sh_tiles,
-                         s.dosrc, s.nptsp, s.ld, s.nptsp, p.npts);
-  else
-    launch_sh_to_do(s.stream, s.S, s.Y, s.ext, s.dosrc, s.nptsp, s.ldo, s.ld, s.nptsp, p.npts,
-                    p.nang);
-  enqueue_sh_to_do_qu(s, nullptr);
+  TRY(ensure_sweep(s, err));
+  enqueue_sh_to_do(s, nullptr);
   (void)hipEventRecord(s.ev[2], s.stream);
   TRY(run_sweeps(s, err));
   (void)hipEventRecord(s.ev[3], s.stream);
@@ -1375,7 +1568,7 @@ static int host_iteration(State& s, bool& fixsh, float& a, int verbose, std::str
   s.tsum[2] += ms[2];  // sweeps (both hemispheres, surface boundary)
   s.tsum[3] += ms[3];  // DO -> SH
   s.tsum[4] += ms[4];  // source (with the next truncation) + reduction
-  if (ring_active(s)) {
+  if (ring_active(s) || planes_active(s)) {
     float a0 = 0.f, a1 = 0.f;
     (void)hipEventElapsedTime(&a0, s.ev[2], s.ev_sweep[1]);
     (void)hipEventElapsedTime(&a1, s.ev_sweep[2], s.ev[3]);
@@ -1516,7 +1709,7 @@ int state_solve(State& s, int maxiter, int verbose, std::string& err) {
   // k_sweep_columns (grids beyond both, and the test options) iterates from
   // the host
   if (s.iters < maxiter && s.solcrit > p.d.solacc) TRY(ensure_sweep(s, err));
-  if (s.use_iter_graph && !verbose && (ring_active(s) || chain_active(s)) && s.iters < maxiter && s.solcrit > p.d.solacc) {
+  if (s.use_iter_graph && !verbose && (planes_active(s) || ring_active(s) || chain_active(s)) && s.iters < maxiter && s.solcrit > p.d.solacc) {
     TRY(state_solve_graph(s, maxiter, err));
     s.last_solve_graph = true;
     launch_fluxes(s.stream, s.dorad, s.nptsp, s.col_of_ref_d, s.fluxw, s.ndown, p.nang, p.npts, s.fluxes);

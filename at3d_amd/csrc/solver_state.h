@@ -117,11 +117,23 @@ struct State {
   int* ngeneral_d = nullptr;
   int4* sh_tiles = nullptr;
   int n_sh_tiles = 0;
+  // plane-ordered sweep (sweep_planes.hip), on grids that take it
+  bool planes_ok = false;
+  PlaneArgs planes;
+  int plane_mz = 0, plane_ms = 0;   // points of a plane across z, of the largest across x or y (0: not in use)
+  size_t plane_lds = 0;
+  int32_t* plane_perm = nullptr;   // [3][nptsp] position -> point
+  int32_t* plane_cols = nullptr;   // columns by axis, the SH->DO tiles' lists
+  int4 *plane_tiles = nullptr, *plane_tiles_qu = nullptr;
+  int n_plane_tiles = 0;
+  std::vector<int32_t> plane_perm_h;
+  std::vector<int8_t> plane_type_h;
+  bool ring_tried = false;     // setup_ring has run (the ring layout is made when something needs it)
   // point-ordered sweep from per-ordinate records (sweep_chain.hip), made on
   // the point-ordered sweep's first use: 0 not yet, 1 ready, -1 not available
   int chain = 0;
   ChainArrays chain_arrays;
-  bool dosrc_level_order = false;   // layout of dosrc written by the last SH->DO
+  int dosrc_order = 0;   // layout of dosrc written by the last SH->DO: 0 points, 1 the ring's, 2 planes
   // options
   int force_general = 0;  // 1: every point through the general characteristic trace
   int use_graph = 1;      // replay the sweep level launches from a HIP graph
@@ -233,5 +245,12 @@ int state_solve(State& s, int maxiter, int verbose, std::string& err);
 // (on) or of (radiance, source) pairs where they fit (off); the captured
 // graphs are dropped.  The solution is kept.
 int state_set_ring4(State& s, bool on, std::string& err);
+// Which sweep the state's options select: the plane-ordered one, the ring, or
+// neither (the point-ordered sweeps).
+bool planes_active(const State& s);
+bool ring_active(const State& s);
+bool ring_wants_radiances_alone(const State& s);
+// The ring's layout where it has not been made yet.
+int ensure_ring(State& s, std::string& err);
 
 }  // namespace at3d

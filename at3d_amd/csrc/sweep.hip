@@ -10,7 +10,9 @@
 // between levels, so a hemisphere's sweep is one launch whose workgroups run
 // independently.
 //
-// k_sweep_ring is the production sweep.  Everything about a one-cell
+// k_sweep_ring sweeps open grids whose planes are past the plane-ordered
+// sweep's largest (sweep_planes.hip) or whose layers are too uneven for it.
+// Everything about a one-cell
 // characteristic that stays fixed during a solve (face points, bilinear
 // weights, transmission, the source-integral coefficients) is computed once
 // per solve by k_sweep_records and stored in level order, so a level is read
@@ -25,6 +27,7 @@
 #include <hip/hip_runtime.h>
 #include <limits.h>
 
+#include "cell_coefs.h"
 #include "kernels.h"
 #include "ring_plan.h"
 
@@ -387,55 +390,6 @@ __device__ inline void sweep_record(const SweepArgs& a, int o, int col, int jl) 
     }
   }
   const_cast<uint4*>(a.rec)[(size_t)col * a.npts + jl] = *reinterpret_cast<const uint4*>(&r);
-}
-
-// Barrier that orders LDS traffic only: outstanding global loads (the next
-// levels' records) and stores (radiances) stay in flight across it.
-__device__ inline void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-
-// The cell integral of a one-cell step (shdomsub1.f:3948-3987, with the
-// reference's tau branches) as coefficients of the face and point sources:
-// src x abs = b0 SRCEXT0 + b1 SRCEXT1 before the clamp at zero, and the
-// cell's transmission, in single precision from the face and point
-// extinctions and the path length.
-__device__ inline void cell_coefs(float ext0, float ext1, float so, float& b0, float& b1, float& trc) {
-  const float e = 0.5f * (ext0 + ext1);
-  const float tau = e * so;
-  float absc;
-  if (tau >= 0.5f) {
-    trc = __expf(-tau);
-    absc = 1.0f - trc;
-  } else {
-    absc = tau * (1.0f - 0.5f * tau * (1.0f - 0.33333333333f * tau * (1.0f - 0.25f * tau)));
-    trc = 1.0f - absc;
-  }
-  float c0, c1;
-  if (tau <= 2.0f) {
-    if (e == 0.0f) {
-      c0 = c1 = 0.0f;
-    } else {
-      const float k = 0.08333333333f * so, re = __builtin_amdgcn_rcpf(e);
-      c0 = (0.5f - k * ext1) * re;
-      c1 = (0.5f + k * ext0) * re;
-    }
-  } else {
-    float e0p = ext0, sc = 1.0f;
-    if (tau > 4.0f) {
-      e0p = ext1 + (ext0 - ext1) * 4.0f / tau;
-      if (ext0 > 0.0f) sc = e0p / ext0;
-    }
-    const float d = e0p + ext1;
-    const float g = 2.0f / d * (1.0f - 2.0f / tau + 2.0f * trc / absc);
-    c0 = sc * (1.0f - ext1 * g) / d;
-    c1 = (1.0f + e0p * g) / d;
-  }
-  b0 = c0 * absc;
-  b1 = c1 * absc;
 }
 
 constexpr uint32_t RECORD_PT_MASK = (1u << RECORD_PT_BITS) - 1;

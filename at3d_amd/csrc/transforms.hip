@@ -129,8 +129,8 @@ __global__ __launch_bounds__(256) void k_sh_to_do(const float* __restrict__ S,
 }
 
 // SH->DO in the sweep's level order: one workgroup computes 64 consecutive
-// positions of one octant's order (S rows gathered through perm) for up to 48
-// columns of that octant; each wave owns 16 positions x 48 columns (three
+// positions of one octant's (or axis's) order (S rows gathered through perm) for
+// up to 48 of its columns; each wave owns 16 positions x 48 columns (three
 // 16x16 MFMA blocks).  S is zero beyond each point's source truncation ns
 // (COMPUTE_SOURCE keeps NS terms, shdomsub1.f:967-1611), so the K loop stops
 // at the largest ns of the tile's rows, rounded up to TK: the terms skipped
@@ -145,6 +145,7 @@ __global__ __launch_bounds__(256) void k_sh_to_do_perm(const float* __restrict__
                                                        const int* __restrict__ ns,
                                                        const int32_t* __restrict__ oct_perm,
                                                        const int4* __restrict__ tiles,
+                                                       const int32_t* __restrict__ cols,
                                                        float* __restrict__ out, int ld, int ldp,
                                                        int npts, const int* __restrict__ stop,
                                                        size_t plane) {
@@ -154,7 +155,8 @@ __global__ __launch_bounds__(256) void k_sh_to_do_perm(const float* __restrict__
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int4 tile = tiles[blockIdx.y];
   const int32_t* perm = oct_perm + (size_t)tile.x * ldp;
-  const int c0 = tile.y, nc = tile.z;
+  const int nc = tile.z;
+  auto column = [&](int j) { return (cols ? cols[tile.y + j] : tile.y + j) + tile.w; };
   const int m0 = blockIdx.x * TM;
   // every wave reduces the same 64 rows: the K extent is uniform in the block
   int kn;
@@ -169,7 +171,7 @@ __global__ __launch_bounds__(256) void k_sh_to_do_perm(const float* __restrict__
   const int lr = tid >> 2, lc = (tid & 3) * 4;
   const float* arow = S + (size_t)perm[m0 + lr] * ld + lc;
   const bool bload = lr < nc;  // threads 0..4*nc-1 load the column tile
-  const float* brow = Yc + (size_t)(c0 + (bload ? lr : 0)) * (QU ? 2 * ld : ld) + lc;
+  const float* brow = Yc + (size_t)column(bload ? lr : 0) * (QU ? 2 * ld : ld) + lc;
   // step kk of the K loop: term kk of the Q plane, or kk - kn of the U plane
   const int kend = QU ? 2 * kn : kn;
   auto aptr = [&](int kk) { return (QU && kk >= kn) ? arow + plane + (kk - kn) : arow + kk; };
@@ -226,7 +228,7 @@ __global__ __launch_bounds__(256) void k_sh_to_do_perm(const float* __restrict__
       o.z = fmaxf(acc[j][2], 0.0f) * e[2];
       o.w = fmaxf(acc[j][3], 0.0f) * e[3];
     }
-    *reinterpret_cast<float4*>(out + (size_t)(c0 + c) * ldp + q0) = o;
+    *reinterpret_cast<float4*>(out + (size_t)column(c) * ldp + q0) = o;
   }
 }
 
@@ -340,19 +342,19 @@ void launch_sh_dot(hipStream_t st, const float* S, const float* Yd, float* raw, 
 }
 
 void launch_sh_to_do_perm(hipStream_t st, const float* S, const float* Yc, const float* ext,
-                          const int* ns, const int32_t* oct_perm, const int4* tiles, int ntiles,
+                          const int* ns, const int32_t* oct_perm, const int4* tiles, const int32_t* cols, int ntiles,
                           float* dosrc, int mp, int ld, int ldp, int npts, const int* stop) {
   if (ntiles <= 0) return;
   dim3 grid(mp / TM, ntiles);
-  k_sh_to_do_perm<false><<<grid, 256, 0, st>>>(S, Yc, ext, ns, oct_perm, tiles, dosrc, ld, ldp, npts, stop, 0);
+  k_sh_to_do_perm<false><<<grid, 256, 0, st>>>(S, Yc, ext, ns, oct_perm, tiles, cols, dosrc, ld, ldp, npts, stop, 0);
 }
 
 void launch_sh_to_do_perm_qu(hipStream_t st, const float* S, size_t plane, const float* Yc, const float* ext,
-                             const int* ns, const int32_t* oct_perm, const int4* tiles, int ntiles,
-                             float* dosrc, int mp, int ld, int ldp, int npts, const int* stop) {
+                             const int* ns, const int32_t* oct_perm, const int4* tiles, const int32_t* cols,
+                             int ntiles, float* dosrc, int mp, int ld, int ldp, int npts, const int* stop) {
   if (ntiles <= 0) return;
   dim3 grid(mp / TM, ntiles);
-  k_sh_to_do_perm<true><<<grid, 256, 0, st>>>(S, Yc, ext, ns, oct_perm, tiles, dosrc, ld, ldp, npts, stop,
+  k_sh_to_do_perm<true><<<grid, 256, 0, st>>>(S, Yc, ext, ns, oct_perm, tiles, cols, dosrc, ld, ldp, npts, stop,
                                               plane);
 }
 
