@@ -199,20 +199,18 @@ struct PlaneArgs {
   const uint16_t* pidx = nullptr;     // [3][npts] natural index of each position of a source row
   const float* ext = nullptr;         // [3][npts] extinction, plane by plane, natural order
   double dx = 0, dy = 0;              // horizontal spacings
+  int sb[3] = {};                     // rows a strip of each axis's planes
 };
-// Largest plane: four points a thread of 1024.  With more a thread's registers
-// spill, and the ring is as fast or faster (96 x 96 x 48, ten points a thread:
-// 1012 us a hemisphere against the ring's 984; 128 x 128 x 64 polarized, 16:
-// 16.8 against 5.8 ms).  LDS bytes for planes of mz points across z and ms
-// across x or y.
-constexpr int PLANE_POINTS_MAX = 4096;
-inline size_t plane_lds_bytes(int mz, int ms, int nz) { return ((size_t)(mz > ms ? mz : ms) + nz) * 16; }
-int sweep_planes_max_lds(int mz, int ms, size_t lds);
+// Largest plane in one piece, and largest strip of others: four and three points
+// a thread of 1024, what their registers hold (strips of four spill 52).
+constexpr int PLANE_POINTS_MAX = 4096, PLANE_STRIP_MAX = 3072;
+// Planes (strips of planes) of mz points across z and ms across x or y.
+int sweep_planes_max_lds(int mz, int ms, bool strips, size_t lds);
 void launch_plane_ext(hipStream_t st, const float* ext, float* out, int nx, int ny, int nz);
 // Columns col0 .. col0+ncol-1 with their boundary radiances (a.qu_only_from as
 // for the ring).
 void launch_sweep_planes(hipStream_t st, const SweepArgs& a, const PlaneArgs& p, int col0, int ncol, int mz, int ms,
-                         size_t lds);
+                         bool strips, size_t lds);
 // ---- sweep_chain.hip: point-ordered sweep from per-ordinate records ------
 // Arrays of one state, rows of npts entries per column: in the octant's list
 // order (q while the levels are made), then in the ordinate's level order.

@@ -422,9 +422,16 @@ int ensure_ring(State& s, std::string& err) { return s.ring_tried ? AT3D_OK : se
 // + 4 where an open side's own plane is swept by the other horizontal axis.
 // False where the plane-ordered sweep does not apply: periodic or refined
 // grids, ordinates whose axis (or an open side's) changes from layer to layer,
-// planes beyond PLANE_POINTS_MAX.  Steps of equal length (a shared edge) may go
+// planes whose strips do not fit in LDS.  Steps of equal length (a shared edge) may go
 // by either face.
-static bool plane_types(const Plan& p, std::vector<int8_t>& type, int& mz, int& ms) {
+struct PlaneTypes {
+  std::vector<int8_t> type;
+  int mz = 0, ms = 0;     // points of the largest strip across z, across x or y
+  int sb[3] = {};         // rows a strip of each axis
+  bool strips = false;    // any plane of more than one
+  size_t lds = 0;
+};
+static bool plane_types(const Plan& p, PlaneTypes& q) {
   if (!p.treeptr.empty() || (p.bcflag & 3) != 3 || p.ipflag != 0) return false;
   if (p.nx1 < 2 || p.ny1 < 2 || p.nz < 2) return false;
   const double dx = ((double)p.xgrid[p.nx1 - 1] - p.xgrid[0]) / (p.nx1 - 1);
@@ -438,37 +445,55 @@ static bool plane_types(const Plan& p, std::vector<int8_t>& type, int& mz, int& 
   if (!(zmin > 0.0) || !(dx > 0.0) || !(dy > 0.0)) return false;
   // (equal to the rounding of the grid's coordinates)
   const double eps = 1e-5;
-  type.assign(p.nang, 0);
-  mz = ms = 0;
+  q.type.assign(p.nang, 0);
+  bool used[3] = {};
   for (int k = 0; k < p.nang; k++) {
     const OrdGeom& g = p.ords[k].g;
     const double hx = dx * fabs(g.cxinv), hy = dy * fabs(g.cyinv);
     const double z0 = zmin * fabs(g.czinv), z1 = zmax * fabs(g.czinv);
     const double hb = std::min(hx, hy);
     if (z1 <= hb * (1 + eps)) {
-      type[k] = 0;
-      mz = p.nx1 * p.ny1;
+      used[0] = true;
       continue;
     }
     if (hb > z0 * (1 + eps)) return false;   // z in some layers only
-    type[k] = hx <= hy ? 1 : 2;
-    ms = std::max(ms, p.nz * (hx <= hy ? p.ny1 : p.nx1));
+    q.type[k] = hx <= hy ? 1 : 2;
+    used[q.type[k]] = true;
     const double ho = std::max(hx, hy);   // the other horizontal axis, in the side's own plane
     if (z1 <= ho * (1 + eps)) continue;
     if (ho > z0 * (1 + eps)) return false;
-    type[k] |= 4;
+    q.type[k] |= 4;
   }
-  return std::max(mz, ms) <= PLANE_POINTS_MAX && plane_lds_bytes(mz, ms, p.nz) <= (size_t)GFX950_LDS_BYTES;
+  // strips of equal rows
+  const int na[3] = {p.ny1, p.nz, p.nz}, nb[3] = {p.nx1, p.ny1, p.nx1}, n[3] = {p.nz, p.nx1, p.ny1};
+  for (int t = 0; t < 3; t++)
+    if (used[t] && na[t] * nb[t] > PLANE_POINTS_MAX) q.strips = true;
+  for (int t = 0; t < 3; t++) {
+    const int most = std::max(1, (q.strips ? PLANE_STRIP_MAX : PLANE_POINTS_MAX) / na[t]);
+    const int ns = (nb[t] + most - 1) / most;
+    q.sb[t] = (nb[t] + ns - 1) / ns;
+    if (!used[t]) continue;
+    if (ns > 1 && na[t] > 1024) return false;   // a thread keeps one line of a strip's last row
+    int& m = t == 0 ? q.mz : q.ms;
+    m = std::max(m, na[t] * q.sb[t]);
+    // the levels' steps, the points, the row before and what is kept of it
+    q.lds = std::max(q.lds, ((size_t)p.nz + na[t] * (q.sb[t] + q.strips)) * 16 + (ns > 1 ? (size_t)na[t] * n[t] * 8 : 0));
+  }
+  return q.lds <= (size_t)GFX950_LDS_BYTES;
 }
 
 // The plane-ordered sweep's orders: per axis the points plane by plane, within
 // a plane grouped by source class (ascending on even planes, descending on odd
 // ones, so classes meet across planes too), and the SH->DO tiles of its columns.
 static int setup_planes(const Plan& p, State& s, std::string& err) {
-  std::vector<int8_t> type;
-  if (!plane_types(p, type, s.plane_mz, s.plane_ms)) return AT3D_OK;
-  s.plane_lds = plane_lds_bytes(s.plane_mz, s.plane_ms, p.nz);
-  if (sweep_planes_max_lds(s.plane_mz, s.plane_ms, s.plane_lds) != 0) {
+  PlaneTypes q;
+  if (!plane_types(p, q)) return AT3D_OK;
+  const std::vector<int8_t>& type = q.type;
+  s.plane_lds = q.lds;
+  s.plane_mz = q.mz;
+  s.plane_ms = q.ms;
+  s.plane_strips = q.strips;
+  if (sweep_planes_max_lds(q.mz, q.ms, q.strips, q.lds) != 0) {
     (void)hipGetLastError();
     return AT3D_OK;
   }
@@ -479,26 +504,34 @@ static int setup_planes(const Plan& p, State& s, std::string& err) {
   const std::vector<int32_t>& cls = p.medium_on_device ? s.medium_cls_h : own;
   s.plane_perm_h.assign((size_t)3 * s.nptsp, 0);
   std::vector<uint16_t> pidx(3 * np, 0);
-  const int nk[3] = {nz, nx, ny}, m[3] = {nx * ny, ny * nz, nx * nz};
+  const int na[3] = {ny, nz, nz}, nb[3] = {nx, ny, nx};
   const int nplanes = nz + nx + ny;
   parallel_for(nplanes, [&](int j) {
-    const int t = j < nz ? 0 : (j < nz + nx ? 1 : 2), k = j - (t == 0 ? 0 : (t == 1 ? nz : nz + nx)), M = m[t];
+    const int t = j < nz ? 0 : (j < nz + nx ? 1 : 2), k = j - (t == 0 ? 0 : (t == 1 ? nz : nz + nx));
     auto point = [&](int q) {
       if (t == 0) return k + nz * q;                              // q = y + ny x
       if (t == 1) return q + nz * ny * k;                         // q = z + nz y
       const int x = q / nz;
       return q - x * nz + nz * (k + ny * x);                      // q = z + nz x
     };
-    std::vector<int> start(p.ml + 3, 0);
-    auto bin = [&](int q) { return (k & 1) ? p.ml - cls[point(q)] : cls[point(q)]; };
-    for (int q = 0; q < M; q++) start[bin(q) + 1]++;
-    for (int l = 0; l <= p.ml; l++) start[l + 1] += start[l];
-    int32_t* perm = s.plane_perm_h.data() + (size_t)t * s.nptsp + (size_t)k * M;
-    uint16_t* ix = pidx.data() + (size_t)t * np + (size_t)k * M;
-    for (int q = 0; q < M; q++) {
-      const int at = start[bin(q)]++;
-      perm[at] = point(q);
-      ix[at] = (uint16_t)q;
+    const int N = t == 0 ? nz : (t == 1 ? nx : ny);
+    for (int b0 = 0; b0 < nb[t]; b0 += q.sb[t]) {   // strip by strip, plane by plane
+      const int M = na[t] * std::min(q.sb[t], nb[t] - b0), g0 = na[t] * b0;
+      std::vector<int> start(p.ml + 3, 0);
+      auto bin = [&](int i) {
+        const int c = cls[point(g0 + i)];
+        return (k & 1) ? p.ml - c : c;
+      };
+      for (int i = 0; i < M; i++) start[bin(i) + 1]++;
+      for (int l = 0; l <= p.ml; l++) start[l + 1] += start[l];
+      const size_t at0 = (size_t)g0 * N + (size_t)k * M;
+      int32_t* perm = s.plane_perm_h.data() + (size_t)t * s.nptsp + at0;
+      uint16_t* ix = pidx.data() + (size_t)t * np + at0;
+      for (int i = 0; i < M; i++) {
+        const int at = start[bin(i)]++;
+        perm[at] = point(g0 + i);
+        ix[at] = (uint16_t)i;
+      }
     }
   });
   for (int t = 0; t < 3; t++)
@@ -538,6 +571,7 @@ static int setup_planes(const Plan& p, State& s, std::string& err) {
   s.planes.ext = d_ext;
   s.planes.dx = ((double)p.xgrid[nx - 1] - p.xgrid[0]) / (nx - 1);
   s.planes.dy = ((double)p.ygrid[ny - 1] - p.ygrid[0]) / (ny - 1);
+  for (int t = 0; t < 3; t++) s.planes.sb[t] = q.sb[t];
   s.planes_ok = true;
   return AT3D_OK;
 }
@@ -560,9 +594,8 @@ size_t plan_footprint_bytes(const Plan& p) {
   b += npts * 4 * 12;                    // per-point scalars, counts, fluxes, partials
   b += npts * 12 + ncells * 57;          // grid positions, cell topology and flags
   b += npts;                             // boundary points
-  std::vector<int8_t> types;
-  int mz = 0, ms = 0;
-  const bool planes = plane_types(p, types, mz, ms);
+  PlaneTypes pt;
+  const bool planes = plane_types(p, pt);
   if (planes) b += 3 * nptsp * 4 + 3 * npts * (2 + 4);   // plane orders and extinctions
   bool chain = !p.treeptr.empty();
   for (int o = 0; o < 8; o++) chain = chain || (p.oct[o].ring_nlev > 0 && (double)npts / p.oct[o].ring_nlev < 4.0);
@@ -1220,7 +1253,8 @@ static void enqueue_sweeps(State& s, const int* stop = nullptr) {
   } else if (planes) {
     SweepArgs a1 = a;
     if (merge_qu) a1.qu_only_from = s.ndown;
-    launch_sweep_planes(s.stream, a1, s.planes, 0, merge_qu ? p.nang : s.ndown, s.plane_mz, s.plane_ms, s.plane_lds);
+    launch_sweep_planes(s.stream, a1, s.planes, 0, merge_qu ? p.nang : s.ndown, s.plane_mz, s.plane_ms,
+                        s.plane_strips, s.plane_lds);
     (void)hipEventRecord(s.ev_sweep[1], s.stream);
   } else if (chain) {
     launch_sweep_chain(s.stream, a, s.chain_arrays, 0, s.ndown);
@@ -1241,7 +1275,8 @@ static void enqueue_sweeps(State& s, const int* stop = nullptr) {
     (void)hipEventRecord(s.ev_sweep[2], s.stream);
     SweepArgs a2 = a;
     if (merge_qu) a2.nst = 1;
-    launch_sweep_planes(s.stream, a2, s.planes, s.ndown, p.nang - s.ndown, s.plane_mz, s.plane_ms, s.plane_lds);
+    launch_sweep_planes(s.stream, a2, s.planes, s.ndown, p.nang - s.ndown, s.plane_mz, s.plane_ms,
+                        s.plane_strips, s.plane_lds);
   } else if (chain) {
     launch_sweep_chain(s.stream, a, s.chain_arrays, s.ndown, p.nang - s.ndown);
   } else {

@@ -120,7 +120,8 @@ struct State {
   // plane-ordered sweep (sweep_planes.hip), on grids that take it
   bool planes_ok = false;
   PlaneArgs planes;
-  int plane_mz = 0, plane_ms = 0;   // points of a plane across z, of the largest across x or y (0: not in use)
+  int plane_mz = 0, plane_ms = 0;   // points of a strip across z, of the largest across x or y (0: not in use)
+  bool plane_strips = false;        // planes of more than one strip
   size_t plane_lds = 0;
   int32_t* plane_perm = nullptr;   // [3][nptsp] position -> point
   int32_t* plane_cols = nullptr;   // columns by axis, the SH->DO tiles' lists

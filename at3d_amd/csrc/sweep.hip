@@ -10,8 +10,9 @@
 // between levels, so a hemisphere's sweep is one launch whose workgroups run
 // independently.
 //
-// k_sweep_ring sweeps open grids whose planes are past the plane-ordered
-// sweep's largest (sweep_planes.hip) or whose layers are too uneven for it.
+// k_sweep_ring sweeps open grids whose layers are too uneven for the
+// plane-ordered sweep (sweep_planes.hip) or whose planes do not fit in LDS in
+// strips.
 // Everything about a one-cell
 // characteristic that stays fixed during a solve (face points, bilinear
 // weights, transmission, the source-integral coefficients) is computed once

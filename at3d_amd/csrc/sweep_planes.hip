@@ -31,6 +31,14 @@
 // 142 ordinates 153 against 253 us; 32 x 32 x 32, 56 ordinates 37 against 92;
 // 48^3, cold 84 against 156 and no records pass (730 us a solve).  Plane order
 // also feeds SH->DO longer runs of one class: 128 against 153 us at 64 x 64 x 40.
+//
+// Planes past PLANE_POINTS_MAX go in strips of rows, one after the other in the
+// ordinate's direction, each through all planes: a strip reads of the one before
+// only its last row, whose radiances and sources stay in LDS (8 bytes a line and
+// plane).  More points a thread instead spill registers (96 x 96 planes, ten a
+// thread: 1012 us a hemisphere; 128 x 128, 16: 16.8 ms).  Against the ring:
+// 96 x 96 x 48, 142 ordinates, 450 us for 984; 128 x 128 x 64 with three Stokes
+// components 2.18 ms for 5.77.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -58,14 +66,15 @@ struct PlanePoint {
   float2 re;
   float s[2];
 };
-// K points a thread. ZT: an ordinate that goes by z.
-template <int T, int K, bool ZT>
+// K points a thread. ZT: an ordinate that goes by z.  STRIPS: planes of more than
+// one strip.
+template <int T, int K, bool ZT, bool STRIPS>
 __device__ __forceinline__ void sweep_planes(const SweepArgs& a, const PlaneArgs& p, int col, int kst, float4* lds) {
   const OrdGeom og = a.ordg[col];
   const int code = p.col_type[col], t = code & 3;
   const int nx = a.nx1, ny = a.ny1, nz = a.nz;
   const int na = ZT ? ny : nz, nb = ZT ? nx : (t == 1 ? ny : nx), N = ZT ? nz : (t == 1 ? nx : ny);
-  const int M = na * nb;
+  const int sb = STRIPS ? p.sb[t] : nb;   // rows (of na points) a strip
   const int lbit = ZT ? og.bitz : (t == 1 ? og.bitx : og.bity);
   const int abit = ZT ? og.bity : og.bitz, bbit = ZT ? og.bitx : (t == 1 ? og.bity : og.bitx);
   // upwind neighbours: a + ua, b + ub
@@ -75,7 +84,10 @@ __device__ __forceinline__ void sweep_planes(const SweepArgs& a, const PlaneArgs
   const int up = og.bitz;
   const int tid = threadIdx.x;
   float4* tab = lds;   // per z level
-  PlanePoint* P = reinterpret_cast<PlanePoint*>(lds + nz);
+  // the strip's points, and on the side upwind the last strip's row next to it
+  // (of the same planes): radiance and source kept in H, [N][na]
+  PlanePoint* P = reinterpret_cast<PlanePoint*>(lds + nz) + (STRIPS && bbit ? na : 0);
+  float2* H = reinterpret_cast<float2*>(lds + nz + (sb + 1) * na);
   const double cx = fabs(og.cx), cy = fabs(og.cy), cz = fabs(og.cz);
   const double hx = p.dx * fabs(og.cxinv), hy = p.dy * fabs(og.cyinv);
   for (int z = tid; z < nz; z += T) {
@@ -98,212 +110,267 @@ __device__ __forceinline__ void sweep_planes(const SweepArgs& a, const PlaneArgs
   auto boundary = [&](int kc, int b) { return !up ? sky : t == 1 ? bottom(kc, b) : bottom(b, kc); };
   // this thread's points: s = tid + k T (the last one again past the end)
   const int stride = ZT ? 1 : (t == 1 ? ny * nz : nz);   // of the point index from plane to plane
-  uint32_t ea = 0, eb = 0;   // on a side across a (x and y ordinates: on the z boundary), across b
-  int goff[ZT ? 1 : K];
-  float wa[ZT ? 1 : K];
-  // the neighbours' offsets in points: a's in the low half, b's in the high one
-  int nbr[K];
+  const int nstrips = STRIPS ? (nb + sb - 1) / sb : 1;
   __syncthreads();
-#pragma unroll
-  for (int k = 0; k < K; k++) {
-    if (k * T >= M) break;
-    const int s = min(tid + k * T, M - 1), bi = s / na, ai = s - bi * na;
-    ea |= (uint32_t)(ZT ? ai == 0 || ai == na - 1 : ai == zstart) << k;
-    eb |= (uint32_t)(bi == 0 || bi == nb - 1) << k;
-    nbr[k] = (ZT && (ai == 0 || ai == na - 1) ? 0 : ua & 0xffff) | ((bi == 0 || bi == nb - 1 ? 0 : uba) * 65536);
-    if constexpr (!ZT) {
-      goff[k] = t == 1 ? s : ai + nz * ny * bi;
-      wa[k] = ai == zstart ? 0.f : tab[ai].y;
-      if (ai == zstart) nbr[k] &= ~0xffff;   // (a boundary value replaces the sum)
-    }
-  }
-  float sl[K], el[K], ec[K], val[K];
-  uint16_t il[K];
-  auto load = [&](int kc) {
-    const int base = kc * M;
-#pragma unroll
+  for (int strip = 0; strip < nstrips; strip++) {
+    const int b0 = STRIPS ? (bbit ? strip : nstrips - 1 - strip) * sb : 0, rows = STRIPS ? min(sb, nb - b0) : nb;
+    const int M = na * rows, g0 = na * b0;
+    uint32_t ea = 0, eb = 0;   // on a side across a (x and y ordinates: on the z boundary), across b
+    uint32_t el_row = 0;       // in the row that the next strip reads (the last downwind)
+    int goff[ZT ? 1 : K];
+    float wa[ZT ? 1 : K];
+    // the neighbours' offsets in points: a's in the low half, b's in the high one
+    int nbr[K];
+  #pragma unroll
     for (int k = 0; k < K; k++) {
       if (k * T >= M) break;
-      const int s = base + min(tid + k * T, M - 1);
-      sl[k] = at<const float>(se, s);
-      il[k] = at<const uint16_t>(pidx, s);
-      el[k] = at<const float>(ext, s);
-    }
-  };
-  float h1[ZT ? K : 1], h2[ZT ? K : 1], h3[ZT ? K : 1];   // the last three planes' radiances
-  int held = 0;
-  load(k0);
-  for (int L = 0; L < N; L++) {
-    const int kc = k0 + L * kstep, par = L & 1;
-    const bool side = !ZT && (L == 0 || L == N - 1);
-    // the last plane's radiance and extinction (a side's own extinction), this
-    // plane's source
-#pragma unroll
-    for (int k = 0; k < K; k++) {
-      if (k * T >= M) break;
-      const int s = min(tid + k * T, M - 1);
-      if (L > 0 && !side) P[s].re = make_float2(val[k], ec[k]);
-      P[il[k]].s[par] = sl[k];
-      ec[k] = el[k];
-      if constexpr (!ZT)
-        if (side) P[s].re.y = ec[k];
-    }
-    lds_barrier();
-    float bv[ZT ? 1 : K];
-    if constexpr (!ZT) {
-      // boundary radiances on the z boundary of this plane
-#pragma unroll
-      for (int k = 0; k < K; k++) {
-        if (k * T >= M) break;
-        bv[k] = sky;
-        if (up && ((ea >> k) & 1)) bv[k] = boundary(kc, min(tid + k * T, M - 1) / na);
-      }
-    }
-    if (L + 1 < N) load(kc + kstep);
-    if (ZT && L == 0) {
-#pragma unroll
-      for (int k = 0; k < K; k++) {
-        if (k * T >= M) break;
-        val[k] = up ? (kst ? 0.0f : a.bcrad_bot[min(tid + k * T, M - 1)]) : sky;   // s = y + ny x, as they are
-      }
-    } else if (!ZT && side) {
+      const int s = min(tid + k * T, M - 1), bl = s / na, ai = s - bl * na, bi = b0 + bl;
+      ea |= (uint32_t)(ZT ? ai == 0 || ai == na - 1 : ai == zstart) << k;
+      eb |= (uint32_t)(bi == 0 || bi == nb - 1) << k;
+      if constexpr (STRIPS) el_row |= (uint32_t)(tid + k * T < M && bl == (bbit ? rows - 1 : 0)) << k;
+      nbr[k] = (ZT && (ai == 0 || ai == na - 1) ? 0 : ua & 0xffff) | ((bi == 0 || bi == nb - 1 ? 0 : uba) * 65536);
       if constexpr (!ZT) {
-      // a side of the open domain: a two-dimensional sweep in z and the other
-      // axis b.  Every point's source integral (in place of its radiance) and
-      // transmission (of the source no longer needed) first, then the first
-      // wavefront adds the transmitted radiances line by line: a line costs an
-      // LDS round trip and three operations.
-      const bool byb = (code & 4) != 0;
-      const float hb = (float)(t == 1 ? hy : hx);
-#pragma unroll
-      for (int k = 0; k < K; k++) {
-        if (k * T >= M) break;
-        const int s = min(tid + k * T, M - 1), bi = s / na, z = s - bi * na;
-        const bool edge = (eb >> k) & 1, preset = (ea >> k) & 1;
-        // the corner upwind and its neighbour, weight w
-        const bool viab = byb && !edge;
-        const int su = preset ? s : viab ? s + uba : s + uz, du = preset || edge ? 0 : viab ? uz : uba;
-        const float w = edge ? 0.f : tab[z].w;
-        const float so = viab ? hb : (float)(fabs((double)a.zgrid[preset ? z : z + uz] - (double)a.zgrid[z]) * fabs(og.czinv));
-        const float ea0 = P[su].re.y, sa0 = P[su].s[par];
-        const float e0 = fmaf(w, P[su + du].re.y - ea0, ea0);
-        const float s0 = fmaf(w, P[su + du].s[par] - sa0, sa0);
-        float b0, b1, trc;
-        cell_coefs(e0, ec[k], so, b0, b1, trc);
-        const float sv = b0 * s0 + b1 * P[s].s[par];
-        P[s].re.x = preset ? bv[k] : (kst ? sv : fmaxf(0.f, sv));
-        P[s].s[par ^ 1] = preset ? 0.f : trc;
+        goff[k] = t == 1 ? g0 + s : ai + nz * ny * bi;
+        wa[k] = ai == zstart ? 0.f : tab[ai].y;
+        if (ai == zstart) nbr[k] &= ~0xffff;   // (a boundary value replaces the sum)
       }
-      lds_barrier();
-      if (tid < 64) {
-        auto step = [&](int s, int su, int du, float w) {
-          const float r0 = P[su].re.x, r1 = P[su + du].re.x;
-          P[s].re.x = fmaf(P[s].s[par ^ 1], fmaf(w, r1 - r0, r0), P[s].re.x);
-        };
-        if (!byb) {
-          for (int z = zstart - uz; z >= 0 && z < nz; z -= uz) {
-            const float w = tab[z].w;
-            for (int b = tid; b < nb; b += 64) {
-              const bool edge = b == 0 || b == nb - 1;
-              step(z + na * b, z + uz + na * b, edge ? 0 : uba, edge ? 0.f : w);
-            }
-          }
-        } else {
-          if (tid < 2) {
-            const int b = tid ? nb - 1 : 0;
-            for (int z = zstart - uz; z >= 0 && z < nz; z -= uz) step(z + na * b, z + uz + na * b, 0, 0.f);
-          }
-          for (int b = bbit ? 1 : nb - 2; b > 0 && b < nb - 1; b -= ub)
-            for (int z = tid; z < nz; z += 64)
-              if (z != zstart) step(z + na * b, z + na * (b + ub), uz, tab[z].w);
-        }
-      }
-      lds_barrier();
-#pragma unroll
-      for (int k = 0; k < K; k++) {
-        if (k * T >= M) break;
-        val[k] = P[min(tid + k * T, M - 1)].re.x;
-      }
-      }
-    } else {
-      const float4 g = tab[ZT ? kc : 0];
-      const float so = g.x, wz = g.y, wb = g.z;
-#pragma unroll
+    }
+    float sl[K], el[K], ec[K], val[K];
+    uint16_t il[K];
+    auto load = [&](int kc) {
+      // (sources strip by strip, extinctions whole planes)
+      const int base = g0 * N + kc * M, ebase = kc * na * nb + g0;
+  #pragma unroll
       for (int k = 0; k < K; k++) {
         if (k * T >= M) break;
         const int s = min(tid + k * T, M - 1);
-        const float w1 = ZT ? wz : wa[k];
-        const float f3 = w1 * wb, f1 = w1 - f3, f2 = wb - f3, f0 = 1.f - w1 - f2;
-        const int oa = (int)(int16_t)nbr[k], ob = nbr[k] >> 16;
-        const PlanePoint *q0 = P + s, *q1 = q0 + oa, *q2 = q0 + ob, *q3 = q1 + ob;
-        const float2 v0 = q0->re, v1 = q1->re, v2 = q2->re, v3 = q3->re;
-        const float c0 = q0->s[par ^ 1], c1 = q1->s[par ^ 1], c2 = q2->s[par ^ 1], c3 = q3->s[par ^ 1];
-        const float e0 = f0 * v0.y + f1 * v1.y + f2 * v2.y + f3 * v3.y;
-        const float s0 = f0 * c0 + f1 * c1 + f2 * c2 + f3 * c3;
-        const float r0 = f0 * v0.x + f1 * v1.x + f2 * v2.x + f3 * v3.x;
-        float b0, b1, trc;
-        cell_coefs(e0, ec[k], so, b0, b1, trc);
-        const float sv = b0 * s0 + b1 * q0->s[par];
-        val[k] = (kst ? sv : fmaxf(0.f, sv)) + trc * r0;
-        if constexpr (!ZT)
-          if ((ea >> k) & 1) val[k] = bv[k];
+        sl[k] = at<const float>(se, base + s);
+        il[k] = at<const uint16_t>(pidx, base + s);
+        el[k] = at<const float>(ext, ebase + s);
       }
-    }
-    if constexpr (ZT) {
-      held++;
-      const bool flush = L == N - 1 || (kc & 3) == (kstep < 0 ? 0 : 3);
-      auto each = [&](auto&& f) {
-#pragma unroll
-        for (int k = 0; k < K; k++) {
-          if (k * T >= M) break;
-          f(k, (uint32_t)(nz * min(tid + k * T, M - 1) + kc));
-        }
-      };
-      if (flush && held == 4) {
-        each([&](int k, uint32_t o) {
-          Vec4 v;
-          v.x = kstep < 0 ? val[k] : h3[k];
-          v.y = kstep < 0 ? h1[k] : h2[k];
-          v.z = kstep < 0 ? h2[k] : h1[k];
-          v.w = kstep < 0 ? h3[k] : val[k];
-          at<Vec4>(rad, kstep < 0 ? o : o - 3) = v;
-        });
-      } else if (flush) {
-        each([&](int k, uint32_t o) {
-          at<float>(rad, o) = val[k];
-          if (held > 1) at<float>(rad, o - kstep) = h1[k];
-          if (held > 2) at<float>(rad, o - 2 * kstep) = h2[k];
-        });
-      }
-#pragma unroll
-      for (int k = 0; k < K; k++) {
-        h3[k] = h2[k];
-        h2[k] = h1[k];
-        h1[k] = val[k];
-      }
-      if (flush) held = 0;
-    } else {
-#pragma unroll
+    };
+    // The row of the strip before: each line of it is fetched by the thread that
+    // owns the same line of this strip's last row (eh: its extinction), so that
+    // H's entry is read and then written by one thread.
+    const bool halo = STRIPS && strip > 0, last = !STRIPS || strip + 1 == nstrips;
+    const int own_row = (bbit ? rows - 1 : 0) * na, halo_row = bbit ? -na : M;
+    float eh = 0.f;
+    auto load_halo = [&](int kc) {
+      if (!halo || el_row == 0) return;
+  #pragma unroll
+      for (int k = 0; k < K; k++)
+        if ((el_row >> k) & 1)
+          eh = at<const float>(ext, kc * na * nb + g0 + halo_row + tid + k * T - own_row);
+    };
+    float h1[ZT ? K : 1], h2[ZT ? K : 1], h3[ZT ? K : 1];   // the last three planes' radiances
+    int held = 0;
+    load(k0);
+    if (STRIPS && !ZT) load_halo(k0);
+    for (int L = 0; L < N; L++) {
+      const int kc = k0 + L * kstep, par = L & 1;
+      const bool side = !ZT && (L == 0 || L == N - 1);
+      // the last plane's radiance and extinction (a side's own extinction), this
+      // plane's source
+  #pragma unroll
       for (int k = 0; k < K; k++) {
         if (k * T >= M) break;
-        at<float>(rad, (uint32_t)(goff[k] + kc * stride)) = val[k];
+        const int s = min(tid + k * T, M - 1);
+        if (L > 0 && !side) P[s].re = make_float2(val[k], ec[k]);
+        P[il[k]].s[par] = sl[k];
+        ec[k] = el[k];
+        if constexpr (!ZT)
+          if (side) P[s].re.y = ec[k];
+      }
+      if constexpr (STRIPS) {
+        // the plane before (a side's: this plane) of the last strip's row, and this
+        // strip's own for the next one
+        if (el_row && (L > 0 || side)) {
+  #pragma unroll
+          for (int k = 0; k < K; k++) {
+            if (!((el_row >> k) & 1)) continue;
+            const int s = tid + k * T, ai = s - own_row;
+            if (halo) {
+              const float2 h = H[(side ? kc : kc - kstep) * na + ai];
+              P[halo_row + ai].re = make_float2(h.x, eh);
+              P[halo_row + ai].s[side ? par : par ^ 1] = h.y;
+            }
+            if (!last && L > 0) H[(kc - kstep) * na + ai] = make_float2(val[k], P[s].s[par ^ 1]);
+          }
+        }
+      }
+      lds_barrier();
+      float bv[ZT ? 1 : K];
+      if constexpr (!ZT) {
+        // boundary radiances on the z boundary of this plane
+  #pragma unroll
+        for (int k = 0; k < K; k++) {
+          if (k * T >= M) break;
+          bv[k] = sky;
+          if (up && ((ea >> k) & 1)) bv[k] = boundary(kc, b0 + min(tid + k * T, M - 1) / na);
+        }
+      }
+      if (L + 1 < N) {
+        load(kc + kstep);
+        if constexpr (STRIPS) load_halo(!ZT && L + 2 == N ? kc + kstep : kc);
+      }
+      if (ZT && L == 0) {
+  #pragma unroll
+        for (int k = 0; k < K; k++) {
+          if (k * T >= M) break;
+          val[k] = up ? (kst ? 0.0f : a.bcrad_bot[g0 + min(tid + k * T, M - 1)]) : sky;   // y + ny x, as they are
+        }
+      } else if (!ZT && side) {
+        if constexpr (!ZT) {
+        // a side of the open domain: a two-dimensional sweep in z and the other
+        // axis b.  Every point's source integral (in place of its radiance) and
+        // transmission (of the source no longer needed) first, then the first
+        // wavefront adds the transmitted radiances line by line: a line costs an
+        // LDS round trip and three operations.
+        const bool byb = (code & 4) != 0;
+        const float hb = (float)(t == 1 ? hy : hx);
+  #pragma unroll
+        for (int k = 0; k < K; k++) {
+          if (k * T >= M) break;
+          const int s = min(tid + k * T, M - 1), z = s - s / na * na;
+          const bool edge = (eb >> k) & 1, preset = (ea >> k) & 1;
+          // the corner upwind and its neighbour, weight w
+          const bool viab = byb && !edge;
+          const int su = preset ? s : viab ? s + uba : s + uz, du = preset || edge ? 0 : viab ? uz : uba;
+          const float w = edge ? 0.f : tab[z].w;
+          const float so = viab ? hb : (float)(fabs((double)a.zgrid[preset ? z : z + uz] - (double)a.zgrid[z]) * fabs(og.czinv));
+          const float ea0 = P[su].re.y, sa0 = P[su].s[par];
+          const float e0 = fmaf(w, P[su + du].re.y - ea0, ea0);
+          const float s0 = fmaf(w, P[su + du].s[par] - sa0, sa0);
+          float b0, b1, trc;
+          cell_coefs(e0, ec[k], so, b0, b1, trc);
+          const float sv = b0 * s0 + b1 * P[s].s[par];
+          P[s].re.x = preset ? bv[k] : (kst ? sv : fmaxf(0.f, sv));
+          P[s].s[par ^ 1] = preset ? 0.f : trc;
+        }
+        lds_barrier();
+        if (tid < 64) {
+          auto step = [&](int s, int su, int du, float w) {
+            const float r0 = P[su].re.x, r1 = P[su + du].re.x;
+            P[s].re.x = fmaf(P[s].s[par ^ 1], fmaf(w, r1 - r0, r0), P[s].re.x);
+          };
+          if (!byb) {
+            for (int z = zstart - uz; z >= 0 && z < nz; z -= uz) {
+              const float w = tab[z].w;
+              for (int b = tid; b < rows; b += 64) {
+                const bool edge = b0 + b == 0 || b0 + b == nb - 1;
+                step(z + na * b, z + uz + na * b, edge ? 0 : uba, edge ? 0.f : w);
+              }
+            }
+          } else {
+            const int be = (tid ? nb - 1 : 0) - b0;   // the open domain's own columns
+            if (tid < 2 && be >= 0 && be < rows) {
+              const int b = be;
+              for (int z = zstart - uz; z >= 0 && z < nz; z -= uz) step(z + na * b, z + uz + na * b, 0, 0.f);
+            }
+            for (int i = 0; i < rows; i++) {
+              const int b = bbit ? i : rows - 1 - i;
+              if (b0 + b == 0 || b0 + b == nb - 1) continue;
+              for (int z = tid; z < nz; z += 64)
+                if (z != zstart) step(z + na * b, z + na * (b + ub), uz, tab[z].w);
+            }
+          }
+        }
+        lds_barrier();
+  #pragma unroll
+        for (int k = 0; k < K; k++) {
+          if (k * T >= M) break;
+          val[k] = P[min(tid + k * T, M - 1)].re.x;
+        }
+        }
+      } else {
+        const float4 g = tab[ZT ? kc : 0];
+        const float so = g.x, wz = g.y, wb = g.z;
+  #pragma unroll
+        for (int k = 0; k < K; k++) {
+          if (k * T >= M) break;
+          const int s = min(tid + k * T, M - 1);
+          const float w1 = ZT ? wz : wa[k];
+          const float f3 = w1 * wb, f1 = w1 - f3, f2 = wb - f3, f0 = 1.f - w1 - f2;
+          const int oa = (int)(int16_t)nbr[k], ob = nbr[k] >> 16;
+          const PlanePoint *q0 = P + s, *q1 = q0 + oa, *q2 = q0 + ob, *q3 = q1 + ob;
+          const float2 v0 = q0->re, v1 = q1->re, v2 = q2->re, v3 = q3->re;
+          const float c0 = q0->s[par ^ 1], c1 = q1->s[par ^ 1], c2 = q2->s[par ^ 1], c3 = q3->s[par ^ 1];
+          const float e0 = f0 * v0.y + f1 * v1.y + f2 * v2.y + f3 * v3.y;
+          const float s0 = f0 * c0 + f1 * c1 + f2 * c2 + f3 * c3;
+          const float r0 = f0 * v0.x + f1 * v1.x + f2 * v2.x + f3 * v3.x;
+          float b0, b1, trc;
+          cell_coefs(e0, ec[k], so, b0, b1, trc);
+          const float sv = b0 * s0 + b1 * q0->s[par];
+          val[k] = (kst ? sv : fmaxf(0.f, sv)) + trc * r0;
+          if constexpr (!ZT)
+            if ((ea >> k) & 1) val[k] = bv[k];
+        }
+      }
+      if constexpr (ZT) {
+        held++;
+        const bool flush = L == N - 1 || (kc & 3) == (kstep < 0 ? 0 : 3);
+        auto each = [&](auto&& f) {
+  #pragma unroll
+          for (int k = 0; k < K; k++) {
+            if (k * T >= M) break;
+            f(k, (uint32_t)(nz * (g0 + min(tid + k * T, M - 1)) + kc));
+          }
+        };
+        if (flush && held == 4) {
+          each([&](int k, uint32_t o) {
+            Vec4 v;
+            v.x = kstep < 0 ? val[k] : h3[k];
+            v.y = kstep < 0 ? h1[k] : h2[k];
+            v.z = kstep < 0 ? h2[k] : h1[k];
+            v.w = kstep < 0 ? h3[k] : val[k];
+            at<Vec4>(rad, kstep < 0 ? o : o - 3) = v;
+          });
+        } else if (flush) {
+          each([&](int k, uint32_t o) {
+            at<float>(rad, o) = val[k];
+            if (held > 1) at<float>(rad, o - kstep) = h1[k];
+            if (held > 2) at<float>(rad, o - 2 * kstep) = h2[k];
+          });
+        }
+  #pragma unroll
+        for (int k = 0; k < K; k++) {
+          h3[k] = h2[k];
+          h2[k] = h1[k];
+          h1[k] = val[k];
+        }
+        if (flush) held = 0;
+      } else {
+  #pragma unroll
+        for (int k = 0; k < K; k++) {
+          if (k * T >= M) break;
+          at<float>(rad, (uint32_t)(goff[k] + kc * stride)) = val[k];
+        }
+      }
+      lds_barrier();
+    }
+    if constexpr (STRIPS && !ZT) {
+      // the last side's row
+      if (el_row && !last) {
+  #pragma unroll
+        for (int k = 0; k < K; k++)
+          if ((el_row >> k) & 1)
+            H[(k0 + (N - 1) * kstep) * na + tid + k * T - own_row] = make_float2(val[k], P[tid + k * T].s[(N - 1) & 1]);
       }
     }
-    lds_barrier();
   }
 }
 
 // KZ, KS: points a thread of planes across z, and across x or y.
-template <int T, int KZ, int KS>
+template <int T, int KZ, int KS, bool STRIPS>
 __global__ __launch_bounds__(T) void k_sweep_planes(SweepArgs a, PlaneArgs p, int col0) {
   if (a.stop && *a.stop) return;
   extern __shared__ float4 planes_lds[];
   const int col = col0 + blockIdx.x;
   if (blockIdx.y == 0 && col >= a.qu_only_from) return;
   if ((p.col_type[col] & 3) == 0)
-    sweep_planes<T, KZ, true>(a, p, col, blockIdx.y, planes_lds);
+    sweep_planes<T, KZ, true, STRIPS>(a, p, col, blockIdx.y, planes_lds);
   else
-    sweep_planes<T, KS, false>(a, p, col, blockIdx.y, planes_lds);
+    sweep_planes<T, KS, false, STRIPS>(a, p, col, blockIdx.y, planes_lds);
 }
 
 // The extinction in each axis's plane order (plane by plane, within a plane by
@@ -334,14 +401,15 @@ struct PlaneShape {
   const void* f;
   void (*go)(dim3, size_t, hipStream_t, const SweepArgs&, const PlaneArgs&, int);
 };
-template <int T, int KZ, int KS>
+template <int T, int KZ, int KS, bool STRIPS = false>
 static PlaneShape plane_shape() {
-  return {reinterpret_cast<const void*>(k_sweep_planes<T, KZ, KS>),
+  return {reinterpret_cast<const void*>(k_sweep_planes<T, KZ, KS, STRIPS>),
           [](dim3 g, size_t lds, hipStream_t st, const SweepArgs& a, const PlaneArgs& p, int c0) {
-            k_sweep_planes<T, KZ, KS><<<g, T, lds, st>>>(a, p, c0);
+            k_sweep_planes<T, KZ, KS, STRIPS><<<g, T, lds, st>>>(a, p, c0);
           }};
 }
-static PlaneShape shape_of(int mz, int ms) {
+static PlaneShape shape_of(int mz, int ms, bool strips) {
+  if (strips) return plane_shape<1024, 3, 3, true>();
   const int m = mz > ms ? mz : ms;
   if (m <= 256) return plane_shape<256, 1, 1>();
   if (m <= 512) return plane_shape<512, 1, 1>();
@@ -354,16 +422,16 @@ static PlaneShape shape_of(int mz, int ms) {
   return ms <= 3072 ? plane_shape<1024, 4, 3>() : plane_shape<1024, 4, 4>();
 }
 
-int sweep_planes_max_lds(int mz, int ms, size_t lds) {
-  return hipFuncSetAttribute(shape_of(mz, ms).f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess
+int sweep_planes_max_lds(int mz, int ms, bool strips, size_t lds) {
+  return hipFuncSetAttribute(shape_of(mz, ms, strips).f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess
              ? 0
              : 1;
 }
 
 void launch_sweep_planes(hipStream_t st, const SweepArgs& a, const PlaneArgs& p, int col0, int ncol, int mz, int ms,
-                         size_t lds) {
+                         bool strips, size_t lds) {
   if (ncol <= 0) return;
-  shape_of(mz, ms).go(dim3(ncol, a.nst), lds, st, a, p, col0);
+  shape_of(mz, ms, strips).go(dim3(ncol, a.nst), lds, st, a, p, col0);
 }
 
 }  // namespace at3d

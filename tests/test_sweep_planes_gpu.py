@@ -35,7 +35,16 @@ GRIDS = {
     "uneven_layers_by_z": lambda: _cloud(7, 9, 12, dx=0.5, z=_uneven(12)),
     "l15": lambda: _cloud(17, 15, 12, nmu=16), "shared_edges": lambda: _cloud(12, 12, 12, dx=0.05, dz=0.05, nmu=16),
     "33x31x20": lambda: _cloud(33, 31, 20, dx=0.02, dz=0.03), "45x46x25": lambda: _cloud(45, 46, 25, dx=0.02, dz=0.03),
-    "64x64x9": lambda: _cloud(64, 64, 9, dx=0.02, dz=0.1), "polarized": lambda: pol_blob(nmu=8, nphi=16),
+    "64x64x9": lambda: _cloud(64, 64, 9, dx=0.02, dz=0.1),
+    # planes of several strips: of unequal rows, across z, x and y, all three, of two points to four a thread
+    "strips_66x63x9": lambda: _cloud(66, 63, 9, dx=0.02, dz=0.1),
+    "strips_97x96x6": lambda: _cloud(97, 96, 6, dx=0.2, dz=0.02),
+    "strips_sides": lambda: _cloud(9, 141, 31, dx=0.02, dz=0.09), "strips_by_x": lambda: _cloud(12, 150, 30, dx=0.02, dy=0.05, dz=0.05),
+    "strips_by_y": lambda: _cloud(150, 12, 30, dx=0.05, dy=0.02, dz=0.05),
+    # (1024 rows: a spacing whose multiples FP32 holds; at 0.1 the coordinates' rounding, half an ulp of 102.4
+    # or 4e-5 of a cell, takes the planes to 6.5e-6 and the ring to 8.8e-6)
+    "strips_1024_rows": lambda: _cloud(5, 1024, 2, dx=0.0625), "strips_l15": lambda: _cloud(70, 70, 61, dx=0.02, dz=0.02, nmu=12),
+    "polarized": lambda: pol_blob(nmu=8, nphi=16),
 }
 
 
@@ -57,7 +66,7 @@ def test_planes_match_point_order(name):
 
 def test_grids_the_planes_do_not_take_keep_their_sweep():
     """Ordinates that go by z in thin layers and by a side in thick ones take
-    the ring, as do planes past the largest, and periodic grids the point
+    the ring, as do strips of one long line, and periodic grids the point
     order; all are what they were."""
     w = _cloud(7, 8, 9, dx=0.05, z=0.4 + 0.9 * (np.arange(9) / 8.0) ** 2.5)
     a, b = S.make_rte(w), S.make_rte(w)
@@ -66,7 +75,7 @@ def test_grids_the_planes_do_not_take_keep_their_sweep():
         r.solve(3, verbose=False)
     assert a.timing("sweep_planes") == 0.0 and a.timing("sweep_ring") == 1.0
     assert rel_l2(a.state_array("do_radiance"), b.state_array("do_radiance")) < 2e-6
-    d = S.make_rte(_cloud(65, 64, 5))
+    d = S.make_rte(_cloud(4, 1100, 3, dx=0.3, dz=0.03))
     d.solve(1, verbose=False)
     assert d.timing("sweep_planes") == 0.0 and d.timing("sweep_ring") == 1.0
     w.bc = "periodic"
