@@ -641,6 +641,14 @@ int at3d_state_set_option(at3d_state* st, const char* key, int32_t value, char* 
     if (rc) set_err(err, errlen, e.c_str());
     return rc;
   }
+  if (k == "dense_analysis") {
+    st->s.dense_analysis = value != 0;
+    std::string e;
+    int rc = ensure_dense_analysis(st->s, e);
+    if (!rc) rc = radiance_rows_written(st->s, e);
+    if (rc) set_err(err, errlen, e.c_str());
+    return rc;
+  }
   if (k == "iteration_graph") {
     st->s.use_iter_graph = value ? 1 : 0;
     return AT3D_OK;

@@ -285,7 +285,7 @@ void launch_radiance_truncation(hipStream_t st, const float* R, int ld, const fl
 void launch_compute_source(hipStream_t st, const SourceArgs& a, int nblocks);
 // R[p][J] = R0[p][J] for J < 4, zero for 4 <= J < max(4, nr[p]) (R is zero
 // beyond NR already); then nr[p] = 4.
-void launch_init_radiance(hipStream_t st, float* R, const float* R0, int* nr, int ld, int npts);
+void launch_init_radiance(hipStream_t st, float* R, const float* R0, int* nr, int* rlen, int ld, int npts);
 
 // ---------------------------------------------------------------------------
 // The per-point medium on the device (medium.hip)

@@ -162,6 +162,11 @@ int state_load(State& s, const int32_t* shptr, const float* source, const int32_
       k_expand_sh<<<nb, 256, 0, s.stream>>>(d_rad + nr_tot * k, d_rp, npts, s.nptsp, s.ld, s.R + s.psh * k, s.nr);
     }
     HIPCHK(hipGetLastError());
+    std::string e;
+    if (radiance_rows_written(s, e) != AT3D_OK) {
+      err = e;
+      return AT3D_ERR_DEVICE;
+    }
     HIPCHK(hipMemsetAsync(s.DS, 0, s.psh * nst * sizeof(float), s.stream));
     HIPCHK(hipMemcpyAsync(s.nos, s.ns, npts * sizeof(int), hipMemcpyDeviceToDevice, s.stream));
     HIPCHK(hipMemcpyAsync(s.fluxes, fluxes, 2 * (size_t)npts * 4, hipMemcpyHostToDevice, s.stream));

@@ -576,6 +576,56 @@ static int setup_planes(const Plan& p, State& s, std::string& err) {
   return AT3D_OK;
 }
 
+// DO->SH tables by factors; t.f stays null where the dense product serves.
+static int setup_analysis(const Plan& p, State& s, bool qu, AnalysisTables& t, std::string& err) {
+  if (!build_analysis(p, s.col_of_ref, qu, t) || analysis_max_lds(t) != 0) {
+    (void)hipGetLastError();
+    t.f = nullptr;
+    return AT3D_OK;
+  }
+  int32_t* ints = nullptr;
+  float* floats = nullptr;
+  TRY(upload(s, ints, t.ints.data(), t.ints.size(), err));
+  TRY(upload(s, floats, t.floats.data(), t.floats.size(), err));
+  t.a.ints = ints;
+  t.a.floats = floats;
+  return AT3D_OK;
+}
+
+// R's rows written other than by k_analysis: any term may be nonzero.
+int radiance_rows_written(State& s, std::string& err) {
+  HIPCHK(hipMemsetAsync(s.rlen, 0x3f, (size_t)2 * s.plan->npts * sizeof(int), s.stream));
+  return AT3D_OK;
+}
+
+// The dense DO->SH tables, by device column, zero padded, where they are read
+// (polarized rows of make_sh_tables_pol's elements: [W2 | W6] for a Q ordinate,
+// [W5 | W3] for a U ordinate).
+int ensure_dense_analysis(State& s, std::string& err) {
+  const Plan& p = *s.plan;
+  if ((!s.ana.f || s.dense_analysis) && !s.W) {
+    std::vector<float> W((size_t)s.ldo * s.ld, 0.f);
+    for (int k = 0; k < p.nang; k++)
+      std::copy_n(&p.wmat[(size_t)k * p.nlm], p.nlm, &W[(size_t)s.col_of_ref[k] * s.ld]);
+    TRY(upload(s, s.W, W.data(), W.size(), err));
+  }
+  if (p.nst == 3 && (!s.ana_qu.f || s.dense_analysis) && !s.Wqu) {
+    const size_t row = 2 * (size_t)s.ld;
+    std::vector<float> W((size_t)2 * s.ldo * row, 0.f);
+    auto el = [&](int e, int k) { return &p.wpol[((size_t)e * p.nang + k) * p.nlm]; };
+    for (int k = 0; k < p.nang; k++) {
+      float* q = &W[(size_t)s.col_of_ref[k] * row];
+      float* u = &W[(size_t)(s.ldo + s.col_of_ref[k]) * row];
+      std::copy_n(el(1, k), p.nlm, q);
+      std::copy_n(el(5, k), p.nlm, q + s.ld);
+      std::copy_n(el(4, k), p.nlm, u);
+      std::copy_n(el(2, k), p.nlm, u + s.ld);
+    }
+    TRY(upload(s, s.Wqu, W.data(), W.size(), err));
+  }
+  return AT3D_OK;
+}
+
 // Device bytes a state of this plan allocates (its arrays and the sweep
 // records; not the per-call render and gradient buffers), for admission by
 // memory footprint before anything is allocated.
@@ -584,11 +634,13 @@ size_t plan_footprint_bytes(const Plan& p) {
   const size_t ld = round_up(p.nlm, 64), nptsp = round_up(p.npts, 64), ldo = round_up(p.nang, 64);
   const size_t ml1 = p.ml + 1;
   size_t b = 0;
-  b += 2 * ldo * ld * 4;                 // Y, W
+  const bool ana = analysis_takes(p);
+  b += (ana ? 1 : 2) * ldo * ld * 4;     // Y, W
   b += 256;                              // iteration control block
   b += 3 * nptsp * ld * 4 * p.nst;       // S, R, DS (each Stokes plane)
   b += 2 * nptsp * ldo * 4 * p.nst;      // DO source and radiance
-  if (p.nst == 3) b += 4 * ldo * ld * 4 * 2 + 4 * npts * ml1 * 4;   // Q / U tables, a2 a3 b1 and b1 TMS terms
+  if (p.nst == 3) b += 4 * ldo * ld * 4 * (ana ? 1 : 2) + 4 * npts * ml1 * 4;   // Q / U tables, a2 a3 b1 and b1 TMS terms
+  b += npts * 8;                         // extents of the radiance rows
   b += npts * 16;                        // two-stream radiance terms
   b += 3 * npts * ml1 * 4;               // chi, tc, tms
   b += npts * 4 * 12;                    // per-point scalars, counts, fluxes, partials
@@ -757,22 +809,20 @@ int state_create(const Plan& p, State& s, std::string& err) {
       }
   }
   // transform matrices by device column, zero padded
-  std::vector<float> Y((size_t)s.ldo * s.ld, 0.f), W((size_t)s.ldo * s.ld, 0.f);
+  std::vector<float> Y((size_t)s.ldo * s.ld, 0.f);
   for (int k = 0; k < p.nang; k++) {
     const int c = s.col_of_ref[k];
-    for (int j = 0; j < p.nlm; j++) {
-      Y[(size_t)c * s.ld + j] = p.ymat[(size_t)k * p.nlm + j];
-      W[(size_t)c * s.ld + j] = p.wmat[(size_t)k * p.nlm + j];
-    }
+    for (int j = 0; j < p.nlm; j++) Y[(size_t)c * s.ld + j] = p.ymat[(size_t)k * p.nlm + j];
   }
   TRY(upload(s, s.Y, Y.data(), Y.size(), err));
-  TRY(upload(s, s.W, W.data(), W.size(), err));
+  TRY(setup_analysis(p, s, false, s.ana, err));
+  if (p.nst == 3) TRY(setup_analysis(p, s, true, s.ana_qu, err));
+  TRY(ensure_dense_analysis(s, err));
   if (p.nst == 3) {
-    // the Q / U transform tables by device column (make_sh_tables_pol's
-    // elements): SH->DO rows [Y2 | Y5] for Q, [Y6 | Y3] for U; DO->SH rows
-    // [W2 | W6] for a Q ordinate, [W5 | W3] for a U ordinate
+    // the Q / U synthesis tables by device column (make_sh_tables_pol's
+    // elements): rows [Y2 | Y5] for Q, [Y6 | Y3] for U
     const size_t row = 2 * (size_t)s.ld;
-    std::vector<float> Yq((size_t)2 * s.ldo * row, 0.f), Wq((size_t)2 * s.ldo * row, 0.f);
+    std::vector<float> Yq((size_t)2 * s.ldo * row, 0.f);
     auto el = [&](const std::vector<float>& t, int e, int k, int j) {
       return t[((size_t)e * p.nang + k) * p.nlm + j];
     };
@@ -780,21 +830,14 @@ int state_create(const Plan& p, State& s, std::string& err) {
       const int c = s.col_of_ref[k];
       float* yq = &Yq[(size_t)c * row];
       float* yu = &Yq[(size_t)(s.ldo + c) * row];
-      float* wq = &Wq[(size_t)c * row];
-      float* wu = &Wq[(size_t)(s.ldo + c) * row];
       for (int j = 0; j < p.nlm; j++) {
         yq[j] = el(p.ypol, 1, k, j);
         yq[s.ld + j] = el(p.ypol, 4, k, j);
         yu[j] = el(p.ypol, 5, k, j);
         yu[s.ld + j] = el(p.ypol, 2, k, j);
-        wq[j] = el(p.wpol, 1, k, j);
-        wq[s.ld + j] = el(p.wpol, 5, k, j);
-        wu[j] = el(p.wpol, 4, k, j);
-        wu[s.ld + j] = el(p.wpol, 2, k, j);
       }
     }
     TRY(upload(s, s.Yqu, Yq.data(), Yq.size(), err));
-    TRY(upload(s, s.Wqu, Wq.data(), Wq.size(), err));
     TRY(upload(s, s.chip, p.chip.data(), p.chip.size(), err));
     TRY(upload(s, s.tms5, p.tms5.data(), p.tms5.size(), err));
   }
@@ -816,6 +859,8 @@ int state_create(const Plan& p, State& s, std::string& err) {
   const size_t nsh = (size_t)s.nptsp * s.ld * s.nst, ndo = (size_t)s.nptsp * s.ldo * s.nst;
   TRY(alloc0(s, s.S, nsh, err));
   TRY(alloc0(s, s.R, nsh, err));
+  TRY(alloc_only(s, s.rlen, (size_t)2 * p.npts, err));
+  TRY(radiance_rows_written(s, err));
   TRY(alloc0(s, s.DS, nsh, err));
   TRY(alloc0(s, s.dosrc, ndo, err));
   TRY(alloc0(s, s.dorad, ndo, err));
@@ -1022,6 +1067,7 @@ static int state_replace(State& s, std::shared_ptr<Plan> owned, SplitFields* f, 
   n.use_ring = s.use_ring;
   n.force_general = s.force_general;
   n.force_ring4 = s.force_ring4;
+  n.dense_analysis = s.dense_analysis;
   n.use_graph = s.use_graph;
   n.use_iter_graph = s.use_iter_graph;
   int rc = state_create(q, n, err);
@@ -1156,9 +1202,12 @@ int state_init_solution(State& s, std::string& err) {
   // a state on a refined grid starts again from its base grid
   if (s.own_plan) TRY(state_replace(s, nullptr, nullptr, err));
   const Plan& p = *s.plan;
-  launch_init_radiance(s.stream, s.R, s.R0, s.nr, s.ld, p.npts);
+  launch_init_radiance(s.stream, s.R, s.R0, s.nr, s.rlen, s.ld, p.npts);
   // the two-stream start is unpolarized: Q and U start at zero
-  if (s.nst == 3) HIPCHK(hipMemsetAsync(s.R + s.psh, 0, 2 * s.psh * sizeof(float), s.stream));
+  if (s.nst == 3) {
+    HIPCHK(hipMemsetAsync(s.R + s.psh, 0, 2 * s.psh * sizeof(float), s.stream));
+    HIPCHK(hipMemsetAsync(s.rlen + p.npts, 0, p.npts * sizeof(int), s.stream));
+  }
   launch_compute_source(s.stream, source_args(s, 1, 0), s.nsrc_blocks);
   s.nr_next_fixsh = false;
   HIPCHK(hipGetLastError());
@@ -1199,6 +1248,7 @@ int state_init_solution_from(State& s, State& src, std::string& err) {
   const size_t nsh = (size_t)s.nptsp * s.ld * s.nst;
   HIPCHK(hipStreamSynchronize(src.stream));
   HIPCHK(hipMemcpyAsync(s.R, src.R, nsh * sizeof(float), hipMemcpyDeviceToDevice, s.stream));
+  TRY(radiance_rows_written(s, err));
   HIPCHK(hipMemcpyAsync(s.nr, src.nr, p.npts * sizeof(int), hipMemcpyDeviceToDevice, s.stream));
   HIPCHK(hipMemcpyAsync(s.fluxes, src.fluxes, 2 * (size_t)p.npts * sizeof(float),
                         hipMemcpyDeviceToDevice, s.stream));
@@ -1437,11 +1487,21 @@ static void enqueue_sh_to_do(State& s, const int* stop) {
   enqueue_sh_to_do_qu(s, stop);
 }
 
-static void enqueue_do_to_sh_qu(State& s, const int* stop) {
-  if (s.nst != 3) return;
+// DO->SH of every Stokes component.
+static void enqueue_do_to_sh(State& s, const int* stop) {
   const Plan& p = *s.plan;
-  launch_do_to_sh_qu(s.stream, s.dorad + s.pdo, s.Wqu, s.nr, s.R + s.psh, s.psh, s.nptsp, s.ld, s.ldo, s.nptsp,
-                     p.npts, stop);
+  if (s.ana.f && !s.dense_analysis)
+    launch_analysis(s.stream, s.ana, false, s.dorad, s.nr, s.rlen, s.R, p.nlm, p.mm, s.ld, s.ldo, s.nptsp, p.npts, stop,
+                    0);
+  else
+    launch_do_to_sh(s.stream, s.dorad, s.W, s.nr, s.R, s.nptsp, s.ld, s.ldo, s.nptsp, p.npts, stop);
+  if (s.nst != 3) return;
+  if (s.ana_qu.f && !s.dense_analysis)
+    launch_analysis(s.stream, s.ana_qu, true, s.dorad + s.pdo, s.nr, s.rlen + s.npts, s.R + s.psh, p.nlm, p.mm, s.ld, s.ldo,
+                    s.nptsp, p.npts, stop, s.psh);
+  else
+    launch_do_to_sh_qu(s.stream, s.dorad + s.pdo, s.Wqu, s.nr, s.R + s.psh, s.psh, s.nptsp, s.ld, s.ldo, s.nptsp,
+                       p.npts, stop);
 }
 
 // One iteration under device control (IterCtl): the loop test and FIXSH,
@@ -1457,8 +1517,7 @@ static void enqueue_iteration(State& s) {
   launch_iter_begin(s.stream, s.ctl);
   enqueue_sh_to_do(s, stop);
   enqueue_sweeps(s, stop);
-  launch_do_to_sh(s.stream, s.dorad, s.W, s.nr, s.R, s.nptsp, s.ld, s.ldo, s.nptsp, p.npts, stop);
-  enqueue_do_to_sh_qu(s, stop);
+  enqueue_do_to_sh(s, stop);
   SourceArgs sa = source_args(s, 0, 0);
   sa.ctl = s.ctl;
   launch_compute_source(s.stream, sa, s.nsrc_blocks);
@@ -1470,7 +1529,7 @@ static void enqueue_iteration(State& s) {
 // The sweep configuration a captured graph holds.
 static int iteration_key(const State& s) {
   return (ring_active(s) ? 1 : 0) | (s.force_general ? 2 : 0) | (s.ring_full ? 4 : 0) | (chain_active(s) ? 8 : 0) |
-         (planes_active(s) ? 16 : 0);
+         (planes_active(s) ? 16 : 0) | (s.dense_analysis ? 32 : 0);
 }
 
 // The graph of ITER_BATCH iterations for the NR buffer parity k (0: s.nr is
@@ -1573,8 +1632,7 @@ static int host_iteration(State& s, bool& fixsh, float& a, int verbose, std::str
   (void)hipEventRecord(s.ev[2], s.stream);
   TRY(run_sweeps(s, err));
   (void)hipEventRecord(s.ev[3], s.stream);
-  launch_do_to_sh(s.stream, s.dorad, s.W, s.nr, s.R, s.nptsp, s.ld, s.ldo, s.nptsp, p.npts);
-  enqueue_do_to_sh_qu(s, nullptr);
+  enqueue_do_to_sh(s, nullptr);
   (void)hipEventRecord(s.ev[4], s.stream);
   if (s.solcrit < 0.001f || s.iters > p.d.iterfixsh) fixsh = true;
   launch_compute_source(s.stream, source_args(s, 0, fixsh ? 1 : 0), s.nsrc_blocks);

@@ -9,6 +9,7 @@
 #include <utility>
 #include <vector>
 
+#include "analysis.h"
 #include "devmem.h"
 #include "direct_beam.h"
 #include "host_plan.h"
@@ -59,6 +60,9 @@ struct State {
   // transforms
   float *Y = nullptr, *W = nullptr, *ysun = nullptr;
   int* lofj = nullptr;
+  AnalysisTables ana, ana_qu;   // DO->SH by factors, where the angle set allows it (.f set)
+  bool dense_analysis = false;  // option: the dense product all the same
+  int* rlen = nullptr;          // [2][npts] where the zeros of R's rows begin (I; Q and U)
   // optics
   float *ext = nullptr, *alb = nullptr, *chi = nullptr, *tc = nullptr, *dirflux = nullptr, *f0 = nullptr;
   // SH fields [nptsp][ld]
@@ -249,6 +253,8 @@ int state_set_ring4(State& s, bool on, std::string& err);
 // Which sweep the state's options select: the plane-ordered one, the ring, or
 // neither (the point-ordered sweeps).
 bool planes_active(const State& s);
+int ensure_dense_analysis(State& s, std::string& err);
+int radiance_rows_written(State& s, std::string& err);
 bool ring_active(const State& s);
 bool ring_wants_radiances_alone(const State& s);
 // The ring's layout where it has not been made yet.

@@ -269,14 +269,17 @@ __global__ __launch_bounds__(256) void k_compute_source(SourceArgs a) {
 
 // INIT_RADIANCE's terms into the SH radiance rows: one wavefront per point.
 __global__ __launch_bounds__(256) void k_init_radiance(float* __restrict__ R, const float* __restrict__ R0,
-                                                       int* __restrict__ nr, int ld, int npts) {
+                                                       int* __restrict__ nr, int* __restrict__ rlen, int ld, int npts) {
   const int lane = threadIdx.x & 63;
   const int p = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (p >= npts) return;
-  const int n = min(ld, max(4, nr[p]));
+  const int n = min(ld, max(4, max(nr[p], rlen[p])));
   float* Rp = R + (size_t)p * ld;
   for (int J = lane; J < n; J += 64) Rp[J] = J < 4 ? R0[(size_t)p * 4 + J] : 0.f;
-  if (lane == 0) nr[p] = 4;
+  if (lane == 0) {
+    nr[p] = 4;
+    rlen[p] = 4;
+  }
 }
 
 // Fixed-order reduction of the block partials.
@@ -338,8 +341,8 @@ void launch_compute_source(hipStream_t st, const SourceArgs& a, int nblocks) {
     k_compute_source<8, 1><<<nblocks, 256, 0, st>>>(a);
 }
 
-void launch_init_radiance(hipStream_t st, float* R, const float* R0, int* nr, int ld, int npts) {
-  k_init_radiance<<<(npts + 3) / 4, 256, 0, st>>>(R, R0, nr, ld, npts);
+void launch_init_radiance(hipStream_t st, float* R, const float* R0, int* nr, int* rlen, int ld, int npts) {
+  k_init_radiance<<<(npts + 3) / 4, 256, 0, st>>>(R, R0, nr, rlen, ld, npts);
 }
 
 void launch_reduce_dots(hipStream_t st, const double* partial, int nblocks, double* out,
