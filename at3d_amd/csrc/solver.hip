@@ -476,8 +476,10 @@ static bool plane_types(const Plan& p, PlaneTypes& q) {
     if (ns > 1 && na[t] > 1024) return false;   // a thread keeps one line of a strip's last row
     int& m = t == 0 ? q.mz : q.ms;
     m = std::max(m, na[t] * q.sb[t]);
-    // the levels' steps, the points, the row before and what is kept of it
-    q.lds = std::max(q.lds, ((size_t)p.nz + na[t] * (q.sb[t] + q.strips)) * 16 + (ns > 1 ? (size_t)na[t] * n[t] * 8 : 0));
+    // the levels' steps, the points, the row before and what is kept of it, the
+    // surface radiances of a plane's z boundary
+    q.lds = std::max(q.lds, ((size_t)p.nz + na[t] * (q.sb[t] + q.strips)) * 16 + (ns > 1 ? (size_t)na[t] * n[t] * 8 : 0) +
+                             (size_t)round_up(q.sb[t], 4) * 4);
   }
   return q.lds <= (size_t)GFX950_LDS_BYTES;
 }

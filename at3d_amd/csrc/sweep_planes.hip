@@ -28,7 +28,7 @@
 // the transmission and source weights of cell_coefs, which the ring read from
 // records (8 bytes a point and ordinate each iteration, and a pass of its own
 // per solve to make them).  Per hemisphere, against k_sweep_ring: 64 x 64 x 40,
-// 142 ordinates 153 against 253 us; 32 x 32 x 32, 56 ordinates 37 against 92;
+// 142 ordinates 138 against 253 us; 32 x 32 x 32, 56 ordinates 37 against 92;
 // 48^3, cold 84 against 156 and no records pass (730 us a solve).  Plane order
 // also feeds SH->DO longer runs of one class: 128 against 153 us at 64 x 64 x 40.
 //
@@ -37,8 +37,8 @@
 // only its last row, whose radiances and sources stay in LDS (8 bytes a line and
 // plane).  More points a thread instead spill registers (96 x 96 planes, ten a
 // thread: 1012 us a hemisphere; 128 x 128, 16: 16.8 ms).  Against the ring:
-// 96 x 96 x 48, 142 ordinates, 450 us for 984; 128 x 128 x 64 with three Stokes
-// components 2.18 ms for 5.77.
+// 96 x 96 x 48, 142 ordinates, 405 us for 984; 128 x 128 x 64 with three Stokes
+// components 2.0 ms for 5.77.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -88,6 +88,8 @@ __device__ __forceinline__ void sweep_planes(const SweepArgs& a, const PlaneArgs
   // (of the same planes): radiance and source kept in H, [N][na]
   PlanePoint* P = reinterpret_cast<PlanePoint*>(lds + nz) + (STRIPS && bbit ? na : 0);
   float2* H = reinterpret_cast<float2*>(lds + nz + (sb + 1) * na);
+  // the surface radiances along the plane's z boundary (x and y ordinates)
+  float* B = STRIPS ? reinterpret_cast<float*>(H + (sb < nb ? N * na : 0)) : reinterpret_cast<float*>(lds + nz + sb * na);
   const double cx = fabs(og.cx), cy = fabs(og.cy), cz = fabs(og.cz);
   const double hx = p.dx * fabs(og.cxinv), hy = p.dy * fabs(og.cyinv);
   for (int z = tid; z < nz; z += T) {
@@ -110,6 +112,12 @@ __device__ __forceinline__ void sweep_planes(const SweepArgs& a, const PlaneArgs
   auto boundary = [&](int kc, int b) { return !up ? sky : t == 1 ? bottom(kc, b) : bottom(b, kc); };
   // this thread's points: s = tid + k T (the last one again past the end)
   const int stride = ZT ? 1 : (t == 1 ? ny * nz : nz);   // of the point index from plane to plane
+  // Radiances go out behind the next barrier where a thread stores three or more
+  // single words a plane: 64 x 64 x 40, 138 us a hemisphere for 154, 96 x 96 x 48
+  // 405 for 451; fewer, or a z ordinate's four planes at a time, the other way
+  // (32^3 41 for 37 us, 96 x 96 x 48 468).
+  constexpr bool LATE = !ZT && K >= 3;
+  constexpr int KB = (K + 1) / 2;   // surface radiances a thread: a row has two points at least
   const int nstrips = STRIPS ? (nb + sb - 1) / sb : 1;
   __syncthreads();
   for (int strip = 0; strip < nstrips; strip++) {
@@ -121,7 +129,7 @@ __device__ __forceinline__ void sweep_planes(const SweepArgs& a, const PlaneArgs
     float wa[ZT ? 1 : K];
     // the neighbours' offsets in points: a's in the low half, b's in the high one
     int nbr[K];
-  #pragma unroll
+#pragma unroll
     for (int k = 0; k < K; k++) {
       if (k * T >= M) break;
       const int s = min(tid + k * T, M - 1), bl = s / na, ai = s - bl * na, bi = b0 + bl;
@@ -132,15 +140,15 @@ __device__ __forceinline__ void sweep_planes(const SweepArgs& a, const PlaneArgs
       if constexpr (!ZT) {
         goff[k] = t == 1 ? g0 + s : ai + nz * ny * bi;
         wa[k] = ai == zstart ? 0.f : tab[ai].y;
-        if (ai == zstart) nbr[k] &= ~0xffff;   // (a boundary value replaces the sum)
+        if (ai == zstart) nbr[k] = (nbr[k] & ~0xffff) | bl;   // (a boundary value replaces the sum: its place in B)
       }
     }
-    float sl[K], el[K], ec[K], val[K];
+    float sl[K], el[K], ec[K], val[K], bl[ZT ? 1 : KB];
     uint16_t il[K];
     auto load = [&](int kc) {
       // (sources strip by strip, extinctions whole planes)
       const int base = g0 * N + kc * M, ebase = kc * na * nb + g0;
-  #pragma unroll
+#pragma unroll
       for (int k = 0; k < K; k++) {
         if (k * T >= M) break;
         const int s = min(tid + k * T, M - 1);
@@ -148,6 +156,12 @@ __device__ __forceinline__ void sweep_planes(const SweepArgs& a, const PlaneArgs
         il[k] = at<const uint16_t>(pidx, base + s);
         el[k] = at<const float>(ext, ebase + s);
       }
+      if constexpr (!ZT)   // the surface radiances of the plane's z boundary
+        if (up) {
+#pragma unroll
+          for (int k = 0; k < KB; k++)
+            if (tid + k * T < rows) bl[k] = boundary(kc, b0 + tid + k * T);
+        }
     };
     // The row of the strip before: each line of it is fetched by the thread that
     // owns the same line of this strip's last row (eh: its extinction), so that
@@ -157,64 +171,119 @@ __device__ __forceinline__ void sweep_planes(const SweepArgs& a, const PlaneArgs
     float eh = 0.f;
     auto load_halo = [&](int kc) {
       if (!halo || el_row == 0) return;
-  #pragma unroll
+#pragma unroll
       for (int k = 0; k < K; k++)
         if ((el_row >> k) & 1)
           eh = at<const float>(ext, kc * na * nb + g0 + halo_row + tid + k * T - own_row);
     };
     float h1[ZT ? K : 1], h2[ZT ? K : 1], h3[ZT ? K : 1];   // the last three planes' radiances
     int held = 0;
+    // plane l's radiances (val) out to the point-ordered row
+    auto put = [&](int kc, int l) {
+      if constexpr (ZT) {
+        held++;
+        const bool flush = l == N - 1 || (kc & 3) == (kstep < 0 ? 0 : 3);
+        auto each = [&](auto&& f) {
+#pragma unroll
+          for (int k = 0; k < K; k++) {
+            if (k * T >= M) break;
+            f(k, (uint32_t)(nz * (g0 + min(tid + k * T, M - 1)) + kc));
+          }
+        };
+        if (flush && held == 4) {
+          each([&](int k, uint32_t o) {
+            Vec4 v;
+            v.x = kstep < 0 ? val[k] : h3[k];
+            v.y = kstep < 0 ? h1[k] : h2[k];
+            v.z = kstep < 0 ? h2[k] : h1[k];
+            v.w = kstep < 0 ? h3[k] : val[k];
+            at<Vec4>(rad, kstep < 0 ? o : o - 3) = v;
+          });
+        } else if (flush) {
+          each([&](int k, uint32_t o) {
+            at<float>(rad, o) = val[k];
+            if (held > 1) at<float>(rad, o - kstep) = h1[k];
+            if (held > 2) at<float>(rad, o - 2 * kstep) = h2[k];
+          });
+        }
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+          h3[k] = h2[k];
+          h2[k] = h1[k];
+          h1[k] = val[k];
+        }
+        if (flush) held = 0;
+      } else {
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+          if (k * T >= M) break;
+          at<float>(rad, (uint32_t)(goff[k] + kc * stride)) = val[k];
+        }
+      }
+    };
     load(k0);
     if (STRIPS && !ZT) load_halo(k0);
-    for (int L = 0; L < N; L++) {
+    for (int L = 0; L < N + (LATE || (STRIPS && !ZT)); L++) {   // (past the last plane: its radiances, its row)
       const int kc = k0 + L * kstep, par = L & 1;
       const bool side = !ZT && (L == 0 || L == N - 1);
-      // the last plane's radiance and extinction (a side's own extinction), this
-      // plane's source
-  #pragma unroll
-      for (int k = 0; k < K; k++) {
-        if (k * T >= M) break;
-        const int s = min(tid + k * T, M - 1);
-        if (L > 0 && !side) P[s].re = make_float2(val[k], ec[k]);
-        P[il[k]].s[par] = sl[k];
-        ec[k] = el[k];
+      if (L < N) {
+        // the last plane's radiance and extinction (a side's own extinction), this
+        // plane's source
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+          if (k * T >= M) break;
+          const int s = min(tid + k * T, M - 1);
+          if (L > 0 && !side) P[s].re = make_float2(val[k], ec[k]);
+          P[il[k]].s[par] = sl[k];
+          ec[k] = el[k];
+          if constexpr (!ZT)
+            if (side) P[s].re.y = ec[k];
+        }
         if constexpr (!ZT)
-          if (side) P[s].re.y = ec[k];
-      }
-      if constexpr (STRIPS) {
-        // the plane before (a side's: this plane) of the last strip's row, and this
-        // strip's own for the next one
-        if (el_row && (L > 0 || side)) {
-  #pragma unroll
-          for (int k = 0; k < K; k++) {
-            if (!((el_row >> k) & 1)) continue;
-            const int s = tid + k * T, ai = s - own_row;
-            if (halo) {
-              const float2 h = H[(side ? kc : kc - kstep) * na + ai];
-              P[halo_row + ai].re = make_float2(h.x, eh);
-              P[halo_row + ai].s[side ? par : par ^ 1] = h.y;
-            }
-            if (!last && L > 0) H[(kc - kstep) * na + ai] = make_float2(val[k], P[s].s[par ^ 1]);
+          if (up) {
+#pragma unroll
+            for (int k = 0; k < KB; k++)
+              if (tid + k * T < rows) B[tid + k * T] = bl[k];
           }
+        if constexpr (STRIPS) {
+          // the plane before (a side's: this plane) of the last strip's row, and this
+          // strip's own for the next one
+          if (el_row && (L > 0 || side)) {
+#pragma unroll
+            for (int k = 0; k < K; k++) {
+              if (!((el_row >> k) & 1)) continue;
+              const int s = tid + k * T, ai = s - own_row;
+              if (halo) {
+                const float2 h = H[(side ? kc : kc - kstep) * na + ai];
+                P[halo_row + ai].re = make_float2(h.x, eh);
+                P[halo_row + ai].s[side ? par : par ^ 1] = h.y;
+              }
+              if (!last && L > 0) H[(kc - kstep) * na + ai] = make_float2(val[k], P[s].s[par ^ 1]);
+            }
+          }
+        }
+      } else if constexpr (STRIPS && !ZT) {
+        // the last side's row (before the barrier: the next strip writes P after it)
+        if (el_row && !last) {
+#pragma unroll
+          for (int k = 0; k < K; k++)
+            if ((el_row >> k) & 1)
+              H[(kc - kstep) * na + tid + k * T - own_row] = make_float2(val[k], P[tid + k * T].s[par ^ 1]);
         }
       }
       lds_barrier();
-      float bv[ZT ? 1 : K];
-      if constexpr (!ZT) {
-        // boundary radiances on the z boundary of this plane
-  #pragma unroll
-        for (int k = 0; k < K; k++) {
-          if (k * T >= M) break;
-          bv[k] = sky;
-          if (up && ((ea >> k) & 1)) bv[k] = boundary(kc, b0 + min(tid + k * T, M - 1) / na);
-        }
-      }
+      // (LATE: the last plane's radiances, then the next plane's loads; waiting for
+      // the loads waits for stores between, which so have this plane's arithmetic
+      // to complete)
+      if constexpr (LATE)
+        if (L > 0) put(kc - kstep, L - 1);
+      if (L == N) break;
       if (L + 1 < N) {
         load(kc + kstep);
         if constexpr (STRIPS) load_halo(!ZT && L + 2 == N ? kc + kstep : kc);
       }
       if (ZT && L == 0) {
-  #pragma unroll
+#pragma unroll
         for (int k = 0; k < K; k++) {
           if (k * T >= M) break;
           val[k] = up ? (kst ? 0.0f : a.bcrad_bot[g0 + min(tid + k * T, M - 1)]) : sky;   // y + ny x, as they are
@@ -228,11 +297,12 @@ __device__ __forceinline__ void sweep_planes(const SweepArgs& a, const PlaneArgs
         // LDS round trip and three operations.
         const bool byb = (code & 4) != 0;
         const float hb = (float)(t == 1 ? hy : hx);
-  #pragma unroll
+#pragma unroll
         for (int k = 0; k < K; k++) {
           if (k * T >= M) break;
           const int s = min(tid + k * T, M - 1), z = s - s / na * na;
           const bool edge = (eb >> k) & 1, preset = (ea >> k) & 1;
+        const float bv = up && preset ? B[nbr[k] & 0xffff] : sky;
           // the corner upwind and its neighbour, weight w
           const bool viab = byb && !edge;
           const int su = preset ? s : viab ? s + uba : s + uz, du = preset || edge ? 0 : viab ? uz : uba;
@@ -244,7 +314,7 @@ __device__ __forceinline__ void sweep_planes(const SweepArgs& a, const PlaneArgs
           float b0, b1, trc;
           cell_coefs(e0, ec[k], so, b0, b1, trc);
           const float sv = b0 * s0 + b1 * P[s].s[par];
-          P[s].re.x = preset ? bv[k] : (kst ? sv : fmaxf(0.f, sv));
+          P[s].re.x = preset ? bv : (kst ? sv : fmaxf(0.f, sv));
           P[s].s[par ^ 1] = preset ? 0.f : trc;
         }
         lds_barrier();
@@ -276,7 +346,7 @@ __device__ __forceinline__ void sweep_planes(const SweepArgs& a, const PlaneArgs
           }
         }
         lds_barrier();
-  #pragma unroll
+#pragma unroll
         for (int k = 0; k < K; k++) {
           if (k * T >= M) break;
           val[k] = P[min(tid + k * T, M - 1)].re.x;
@@ -285,13 +355,14 @@ __device__ __forceinline__ void sweep_planes(const SweepArgs& a, const PlaneArgs
       } else {
         const float4 g = tab[ZT ? kc : 0];
         const float so = g.x, wz = g.y, wb = g.z;
-  #pragma unroll
+#pragma unroll
         for (int k = 0; k < K; k++) {
           if (k * T >= M) break;
           const int s = min(tid + k * T, M - 1);
           const float w1 = ZT ? wz : wa[k];
           const float f3 = w1 * wb, f1 = w1 - f3, f2 = wb - f3, f0 = 1.f - w1 - f2;
-          const int oa = (int)(int16_t)nbr[k], ob = nbr[k] >> 16;
+          const bool preset = !ZT && ((ea >> k) & 1);
+          const int oa = preset ? 0 : (int)(int16_t)nbr[k], ob = nbr[k] >> 16;
           const PlanePoint *q0 = P + s, *q1 = q0 + oa, *q2 = q0 + ob, *q3 = q1 + ob;
           const float2 v0 = q0->re, v1 = q1->re, v2 = q2->re, v3 = q3->re;
           const float c0 = q0->s[par ^ 1], c1 = q1->s[par ^ 1], c2 = q2->s[par ^ 1], c3 = q3->s[par ^ 1];
@@ -302,60 +373,11 @@ __device__ __forceinline__ void sweep_planes(const SweepArgs& a, const PlaneArgs
           cell_coefs(e0, ec[k], so, b0, b1, trc);
           const float sv = b0 * s0 + b1 * q0->s[par];
           val[k] = (kst ? sv : fmaxf(0.f, sv)) + trc * r0;
-          if constexpr (!ZT)
-            if ((ea >> k) & 1) val[k] = bv[k];
+          if (preset) val[k] = up ? B[nbr[k] & 0xffff] : sky;
         }
       }
-      if constexpr (ZT) {
-        held++;
-        const bool flush = L == N - 1 || (kc & 3) == (kstep < 0 ? 0 : 3);
-        auto each = [&](auto&& f) {
-  #pragma unroll
-          for (int k = 0; k < K; k++) {
-            if (k * T >= M) break;
-            f(k, (uint32_t)(nz * (g0 + min(tid + k * T, M - 1)) + kc));
-          }
-        };
-        if (flush && held == 4) {
-          each([&](int k, uint32_t o) {
-            Vec4 v;
-            v.x = kstep < 0 ? val[k] : h3[k];
-            v.y = kstep < 0 ? h1[k] : h2[k];
-            v.z = kstep < 0 ? h2[k] : h1[k];
-            v.w = kstep < 0 ? h3[k] : val[k];
-            at<Vec4>(rad, kstep < 0 ? o : o - 3) = v;
-          });
-        } else if (flush) {
-          each([&](int k, uint32_t o) {
-            at<float>(rad, o) = val[k];
-            if (held > 1) at<float>(rad, o - kstep) = h1[k];
-            if (held > 2) at<float>(rad, o - 2 * kstep) = h2[k];
-          });
-        }
-  #pragma unroll
-        for (int k = 0; k < K; k++) {
-          h3[k] = h2[k];
-          h2[k] = h1[k];
-          h1[k] = val[k];
-        }
-        if (flush) held = 0;
-      } else {
-  #pragma unroll
-        for (int k = 0; k < K; k++) {
-          if (k * T >= M) break;
-          at<float>(rad, (uint32_t)(goff[k] + kc * stride)) = val[k];
-        }
-      }
+      if constexpr (!LATE) put(kc, L);
       lds_barrier();
-    }
-    if constexpr (STRIPS && !ZT) {
-      // the last side's row
-      if (el_row && !last) {
-  #pragma unroll
-        for (int k = 0; k < K; k++)
-          if ((el_row >> k) & 1)
-            H[(k0 + (N - 1) * kstep) * na + tid + k * T - own_row] = make_float2(val[k], P[tid + k * T].s[(N - 1) & 1]);
-      }
     }
   }
 }
@@ -417,6 +439,10 @@ static PlaneShape shape_of(int mz, int ms, bool strips) {
   if (mz <= 2048) {
     if (ms <= 2048) return plane_shape<1024, 2, 2>();
     return ms <= 3072 ? plane_shape<1024, 2, 3>() : plane_shape<1024, 2, 4>();
+  }
+  if (mz <= 3072) {
+    if (ms <= 2048) return plane_shape<1024, 3, 2>();
+    return ms <= 3072 ? plane_shape<1024, 3, 3>() : plane_shape<1024, 3, 4>();
   }
   if (ms <= 2048) return plane_shape<1024, 4, 2>();
   return ms <= 3072 ? plane_shape<1024, 4, 3>() : plane_shape<1024, 4, 4>();

@@ -35,6 +35,7 @@ GRIDS = {
     "uneven_layers_by_z": lambda: _cloud(7, 9, 12, dx=0.5, z=_uneven(12)),
     "l15": lambda: _cloud(17, 15, 12, nmu=16), "shared_edges": lambda: _cloud(12, 12, 12, dx=0.05, dz=0.05, nmu=16),
     "33x31x20": lambda: _cloud(33, 31, 20, dx=0.02, dz=0.03), "45x46x25": lambda: _cloud(45, 46, 25, dx=0.02, dz=0.03),
+    "52x53x40": lambda: _cloud(52, 53, 40, dx=0.03, dz=0.02), "55x50x60": lambda: _cloud(55, 50, 60, dx=0.03, dz=0.03),
     "64x64x9": lambda: _cloud(64, 64, 9, dx=0.02, dz=0.1),
     # planes of several strips: of unequal rows, across z, x and y, all three, of two points to four a thread
     "strips_66x63x9": lambda: _cloud(66, 63, 9, dx=0.02, dz=0.1),
