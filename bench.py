@@ -129,7 +129,7 @@ def cpu_gradient(w, rays, meas):
 
 
 # kernel class -> device kernel name in the rocprofv3 counter summaries
-KERNEL_NAMES = {"sweep": "k_sweep_ring", "sh_to_do": "k_sh_to_do_perm", "do_to_sh": "k_do_to_sh",
+KERNEL_NAMES = {"sweep": "k_sweep_planes", "sh_to_do": "k_sh_to_do_perm", "do_to_sh": "k_analysis",
                 "source": "k_compute_source"}
 
 
@@ -256,7 +256,8 @@ def polarized_leg(cpu_runs):
     out = {"workload": "128x128x64 open cloud, NSTOKES 3, NMU16 NPHI32 L15, solacc 1e-4, "
                        "3 wavelengths (0.47 0.66 0.86 um), 9 views of 128x128 I/Q/U",
            "npts": rtes[0].plan_size("npts"),
-           "sweep": ("level-ordered, ring of radiances ({:.0f} KB of LDS)" if rtes[0].timing("sweep_ring4") else
+           "sweep": ("plane-ordered ({:.0f} KB of LDS)" if rtes[0].timing("sweep_planes") else
+                     "level-ordered, ring of radiances ({:.0f} KB of LDS)" if rtes[0].timing("sweep_ring4") else
                      "level-ordered ({:.0f} KB of LDS)").format(rtes[0].timing("sweep_ring_lds") / 1024)
            if rtes[0].timing("sweep_ring") else "point-ordered",
            "iterations": [r.num_iterations for r in rtes], "solve_wall_s": wall,
@@ -529,7 +530,7 @@ def main():
     kern = {}
     n_it = max(kiters, 1)
     # one sweep pass = one launch per hemisphere (a workgroup per ordinate walking
-    # the octant's dependency levels); algorithmic bytes per (ordinate, point):
+    # the grid's planes, or its octant's dependency levels); algorithmic bytes per (ordinate, point):
     # read the DO source and the extinction, write the DO radiance (3 x 4 B)
     sweep_bytes = nang * npts * 12.0
     ms_pass = ksum["sweep"] / n_it
@@ -541,12 +542,14 @@ def main():
                      "ms_per_launch": ms_launch, "bytes_per_launch": sweep_bytes / 2,
                      "GB/s": sweep_bytes / 2 / ms_launch / 1e6,
                      "level_ordered": bool(rte.timing("sweep_ring")),
+                     "plane_ordered": bool(rte.timing("sweep_planes")),
                      "lds_bytes": int(rte.timing("sweep_ring_lds")),
                      "multi_cell_points": int(rte.timing("sweep_general_points"))}
     # the transforms on the terms that can be nonzero (each point's source
-    # truncation NS for SH->DO, radiance truncation NR for DO->SH): useful
-    # flops 2 NANG sum(NS) and 2 NANG sum(NR), bytes one read of those terms,
-    # one read or write of NANG values per point
+    # truncation NS for SH->DO, radiance truncation NR for DO->SH): bytes one
+    # read or write of those terms and of NANG values per point; the flops of a
+    # dense product on them, 2 NANG sum(NS) and 2 NANG sum(NR) (DO->SH goes by
+    # factors and executes fewer)
     for k, cnt in (("sh_to_do", ns), ("do_to_sh", nr)):
         ms = ksum[k] / n_it
         fl = 2.0 * nang * cnt.sum()
