@@ -1,5 +1,5 @@
-// The cell integral of a short characteristic in single precision and the
-// workgroup barrier of the sweeps (device).
+// The cell integral of a short characteristic in single precision, and the
+// workgroup barrier and wavefront fence of the sweeps (device).
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -11,6 +11,16 @@ __device__ inline void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// Orders a wavefront's own LDS traffic: what its lanes wrote before is what its
+// other lanes read after.  The hardware keeps a wavefront's LDS operations in
+// order, so no instruction comes of it; without it nothing keeps the compiler
+// from moving one lane's load over another's store.
+__device__ inline void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
 }
 
 // 1 / x to a last place: the hardware's estimate and one Newton step (3

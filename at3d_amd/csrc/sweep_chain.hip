@@ -25,6 +25,7 @@
 // general trace by 1e-16 before that rounding.
 #include <hip/hip_runtime.h>
 
+#include "cell_coefs.h"
 #include "kernels.h"
 
 namespace at3d {
@@ -100,6 +101,7 @@ __global__ __launch_bounds__(64) void k_chain_levels(SweepArgs a, ChainArrays c)
       l = m;
       if (!__any(changed)) break;
       lev[pt] = (uint16_t)l;
+      wave_lds_fence();
     }
     top = max(top, l);
   }
@@ -202,7 +204,7 @@ constexpr int CHAIN_AHEAD = 6;   // chunks of 64 records in flight
 // chain, 64 records at a time (one per lane, the next CHAIN_AHEAD chunks loading
 // meanwhile): the lanes of one level gather their corners from the LDS row and write their
 // points, then the next level's lanes do; a wavefront's LDS operations are in
-// order, so levels need no barrier.  Bound by levels x (LDS round trip + the
+// order, so levels need no barrier, only a fence for the compiler.  Bound by levels x (LDS round trip + the
 // FP64 sum).  The row is kept in doubles where they fit (four conversions less
 // per level: 0.29 against 0.33 ms at 16^3 periodic).  The other wavefronts help
 // to fill and write out the row.
@@ -246,11 +248,13 @@ __global__ __launch_bounds__(CHAIN_THREADS) void k_sweep_chain(SweepArgs a, Chai
       Row* out = row + (x.ptlev & 0xffff);
       const int lev = p0 + tid < n ? (int)(x.ptlev >> 16) : 0;
       const int l0 = __builtin_amdgcn_readlane(lev, 0), l1 = __builtin_amdgcn_readlane(lev, min(n - p0, 64) - 1);
-      for (int l = l0; l <= l1; l++)
+      for (int l = l0; l <= l1; l++) {
         if (lev == l) {
           const double r1 = *q1, r2 = *q2, r3 = *q3, r4 = *q4;
           *out = (float)(fma(f2, r2, fma(f1, r1, x.r)) + fma(f4, r4, f3 * r3));
         }
+        wave_lds_fence();
+      }
     };
     Rec x[CHAIN_AHEAD];
 #pragma unroll

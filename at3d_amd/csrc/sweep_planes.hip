@@ -330,6 +330,7 @@ __device__ __forceinline__ void sweep_planes(const SweepArgs& a, const PlaneArgs
                 const bool edge = b0 + b == 0 || b0 + b == nb - 1;
                 step(z + na * b, z + uz + na * b, edge ? 0 : uba, edge ? 0.f : w);
               }
+              wave_lds_fence();
             }
           } else {
             const int be = (tid ? nb - 1 : 0) - b0;   // the open domain's own columns
@@ -337,11 +338,13 @@ __device__ __forceinline__ void sweep_planes(const SweepArgs& a, const PlaneArgs
               const int b = be;
               for (int z = zstart - uz; z >= 0 && z < nz; z -= uz) step(z + na * b, z + uz + na * b, 0, 0.f);
             }
+            wave_lds_fence();
             for (int i = 0; i < rows; i++) {
               const int b = bbit ? i : rows - 1 - i;
               if (b0 + b == 0 || b0 + b == nb - 1) continue;
               for (int z = tid; z < nz; z += 64)
                 if (z != zstart) step(z + na * b, z + na * (b + ub), uz, tab[z].w);
+              wave_lds_fence();
             }
           }
         }
