@@ -95,8 +95,10 @@ __global__ __launch_bounds__(64) void k_chain_levels(SweepArgs a, ChainArrays c)
     // (at most 64 times: the list is a topological order)
     int l = 0;
     for (int it = 0; it < 65; it++) {
-      const int m = 1 + max(max((int)lev[q.x & 0xffff], (int)lev[q.x >> 16]),
-                            max((int)lev[q.y & 0xffff], (int)lev[q.y >> 16]));
+      // (a bad trace reads itself and would climb with every turn: no level is
+      // past the number of entries, which the counts and the row are sized for)
+      const int m = min(n, 1 + max(max((int)lev[q.x & 0xffff], (int)lev[q.x >> 16]),
+                                   max((int)lev[q.y & 0xffff], (int)lev[q.y >> 16])));
       const bool changed = m != l;
       l = m;
       if (!__any(changed)) break;
