@@ -1474,14 +1474,19 @@ static void enqueue_sh_to_do_qu(State& s, const int* stop) {
                        s.nptsp, p.npts, stop);
 }
 
+// The layout of dosrc that the active sweep reads (State::dosrc_order).
+static int source_order(const State& s) { return planes_active(s) ? 2 : (ring_active(s) ? 1 : 0); }
+
 // SH->DO of the I rows, in the layout the active sweep reads, then Q and U.
+// (Whoever runs it sets dosrc_order: a captured graph enqueues it once and runs
+// it in later solves.)
 static void enqueue_sh_to_do(State& s, const int* stop) {
   const Plan& p = *s.plan;
-  s.dosrc_order = planes_active(s) ? 2 : (ring_active(s) ? 1 : 0);
-  if (s.dosrc_order == 2)
+  const int order = source_order(s);
+  if (order == 2)
     launch_sh_to_do_perm(s.stream, s.S, s.Y, s.ext, s.ns, s.plane_perm, s.plane_tiles, s.plane_cols, s.n_plane_tiles,
                          s.dosrc, s.nptsp, s.ld, s.nptsp, p.npts, stop);
-  else if (s.dosrc_order == 1)
+  else if (order == 1)
     launch_sh_to_do_perm(s.stream, s.S, s.Y, s.ext, s.ns, s.oct_perm, s.sh_tiles, nullptr, s.n_sh_tiles, s.dosrc,
                          s.nptsp, s.ld, s.nptsp, p.npts, stop);
   else
@@ -1577,6 +1582,7 @@ static int state_solve_graph(State& s, int maxiter, std::string& err) {
   const int parity = s.nr == s.nr_buf0 ? 0 : 1;
   const int key = iteration_key(s);
   if (!s.iter_exec[parity] || s.iter_key[parity] != key) TRY(capture_iterations(s, parity, err));
+  s.dosrc_order = source_order(s);
   // every batch runs ITER_BATCH iterations unless the device stops: the
   // host bound only guards against a control block that never moves
   const int max_batches = (maxiter - s.iters) / State::ITER_BATCH + 2;
@@ -1630,6 +1636,7 @@ static int host_iteration(State& s, bool& fixsh, float& a, int verbose, std::str
   std::swap(s.nr, s.nr_next);
   (void)hipEventRecord(s.ev[0], s.stream);
   TRY(ensure_sweep(s, err));
+  s.dosrc_order = source_order(s);
   enqueue_sh_to_do(s, nullptr);
   (void)hipEventRecord(s.ev[2], s.stream);
   TRY(run_sweeps(s, err));

@@ -85,6 +85,22 @@ def test_grids_the_planes_do_not_take_keep_their_sweep():
     assert c.timing("sweep_planes") == 0.0 and c.timing("sweep_ring") == 0.0
 
 
+def test_do_source_follows_the_sweep_that_wrote_it():
+    """Each sweep has its own order of the DO source rows; they read back by
+    point whichever sweep ran last, also where a graph captured earlier is
+    replayed after iterations launched one by one in another order."""
+    w = _cloud(14, 11, 10, nmu=8)
+    a = S.make_rte(w)
+    got = []
+    for ring, graph in ((1, 1), (0, 0), (1, 1), (2, 1), (1, 0), (2, 1), (1, 1), (0, 1), (1, 1)):
+        a.set_option("sweep_ring", ring)
+        a.set_option("iteration_graph", graph)
+        a.solve(60, verbose=False)
+        got.append(a.state_array("do_source"))
+    for x in got[1:]:
+        assert rel_l2(x, got[0]) < 5e-6
+
+
 def test_options_switch_between_sweeps_on_one_state():
     """Planes, ring, point order and planes again on one state, iterations from
     graphs: each solve is the one a state of its own gives."""
