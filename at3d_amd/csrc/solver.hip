@@ -417,6 +417,24 @@ static int setup_ring(const Plan& p, State& s, std::string& err) {
 
 int ensure_ring(State& s, std::string& err) { return s.ring_tried ? AT3D_OK : setup_ring(*s.plan, s, err); }
 
+// Whether the ring of a plan's grid, at its smallest (radiances alone over the
+// five levels that four-point sectors need, as build_ring_plan lays it out),
+// fits in LDS.
+static bool ring_fits(const Plan& p) {
+  bool used[8] = {};
+  for (const Ordinate& od : p.ords) used[od.g.ioct] = true;
+  int slots = 0, nlev = 0;
+  for (int o = 0; o < 8; o++) {
+    if (!used[o]) continue;
+    const std::vector<int32_t>& off = p.oct[o].ring_off;
+    const int n = (int)off.size() - 1;
+    nlev = std::max(nlev, n);
+    for (int L = 0; L < n; L++) slots = std::max(slots, off[std::min(n, L + 5)] - off[L]);
+  }
+  return slots <= 65536 && p.npts < (1 << RECORD_PT_BITS) && p.nz < 8192 &&
+         ring_lds_bytes(slots, nlev + 2, 0, 4) <= GFX950_LDS_BYTES;
+}
+
 // The axis of every ordinate of a plan (device column order is the caller's):
 // the one whose spacing over direction cosine is the shortest, for every layer;
 // + 4 where an open side's own plane is swept by the other horizontal axis.
@@ -424,6 +442,10 @@ int ensure_ring(State& s, std::string& err) { return s.ring_tried ? AT3D_OK : se
 // grids, ordinates whose axis (or an open side's) changes from layer to layer,
 // planes whose strips do not fit in LDS.  Steps of equal length (a shared edge) may go
 // by either face.
+// Grids whose ring does not fit keep the point order too, whose steps are FP64:
+// the planes' are FP32 like the ring's, and nearer to FP64 than those (do_radiance
+// after three iterations, 15 grids: 1.4e-7 to 5.2e-7 against 2.3e-7 to 2.1e-6),
+// but no grid gives up FP64 steps for them (111 x 109 x 110 on, 160 x 160 x 64).
 struct PlaneTypes {
   std::vector<int8_t> type;
   int mz = 0, ms = 0;     // points of the largest strip across z, across x or y
@@ -433,7 +455,7 @@ struct PlaneTypes {
 };
 static bool plane_types(const Plan& p, PlaneTypes& q) {
   if (!p.treeptr.empty() || (p.bcflag & 3) != 3 || p.ipflag != 0) return false;
-  if (p.nx1 < 2 || p.ny1 < 2 || p.nz < 2) return false;
+  if (p.nx1 < 2 || p.ny1 < 2 || p.nz < 2 || !ring_fits(p)) return false;
   const double dx = ((double)p.xgrid[p.nx1 - 1] - p.xgrid[0]) / (p.nx1 - 1);
   const double dy = ((double)p.ygrid[p.ny1 - 1] - p.ygrid[0]) / (p.ny1 - 1);
   double zmin = 1e300, zmax = 0.0;

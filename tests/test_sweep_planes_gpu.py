@@ -85,6 +85,22 @@ def test_grids_the_planes_do_not_take_keep_their_sweep():
     assert c.timing("sweep_planes") == 0.0 and c.timing("sweep_ring") == 0.0
 
 
+def test_grids_past_the_ring_keep_their_fp64_steps():
+    """A grid whose ring does not fit in LDS sweeps point by point in FP64, also
+    where strips of planes would fit: bit for bit the point-ordered sweep."""
+    rng = np.random.default_rng(3)
+    shape = (111, 109, 110)
+    ext = rng.lognormal(0.0, 0.5, shape).astype(np.float32)
+    w = S.Workload("past_ring", 0.05, 0.05, (0.04 * np.arange(110)).astype(np.float32),
+                   [(ext, np.full(shape, 0.95, np.float32), S.hg_legendre(0.5, 8))], bc="open", nmu=2, nphi=4)
+    a, b = (S.make_rte(w, max_total_mb=50000.0, adapt_grid_factor=1.0) for _ in range(2))
+    b.set_option("sweep_ring", 0)
+    for r in (a, b):
+        r.solve(2, verbose=False)
+    assert a.timing("sweep_planes") == 0.0 and a.timing("sweep_ring") == 0.0
+    assert np.array_equal(a.state_array("do_radiance"), b.state_array("do_radiance"))
+
+
 def test_do_source_follows_the_sweep_that_wrote_it():
     """Each sweep has its own order of the DO source rows; they read back by
     point whichever sweep ran last, also where a graph captured earlier is
