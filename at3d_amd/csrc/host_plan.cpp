@@ -1475,6 +1475,12 @@ int build_plan(const at3d_scene_desc& desc, Plan& p, std::string& err) {
     err = "Insufficient Spherical Harmonics (NLM < 4)";
     return AT3D_ERR_ARG;
   }
+  // NLM counts the terms of M <= L + 1; past that it is smaller than (L + 1)^2,
+  // the terms there are, and every table of NLM entries would be overrun
+  if (p.mm > p.ml + 1) {
+    err = "num_phi_bins must be below 2 num_mu_bins + 4 (the azimuthal order M = num_phi_bins / 2 - 1 would pass L + 1)";
+    return AT3D_ERR_ARG;
+  }
   p.nphi0max = p.nphi;
   p.nleg = d.deltam ? p.ml + 1 : p.ml;
   p.numphase = d.numphase;

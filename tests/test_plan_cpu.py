@@ -118,6 +118,26 @@ def test_unsupported_options_raise():
         S.make_rte(w, transmin=0.5)
 
 
+@pytest.mark.parametrize("nmu,nphi", [(4, 12), (4, 13), (4, 16), (8, 32), (6, 40)])
+def test_more_azimuths_than_the_harmonics_hold_raise(nmu, nphi):
+    """NPHI from 2 NMU + 4 on: NLM falls below the number of terms, and the
+    tables were overrun."""
+    with pytest.raises(_lib.SHDOMError, match="num_phi_bins"):
+        S.make_rte(blob8("open", nmu=nmu, nphi=nphi))
+
+
+@pytest.mark.parametrize("nmu,nphi", [(4, 8), (4, 9), (4, 10), (4, 11), (8, 19)])
+def test_as_many_azimuths_as_the_harmonics_hold(nmu, nphi):
+    """Up to 2 NMU + 3 every term has its place: the tables' inverse on the
+    terms with m = 0, which every zenith angle carries, is the identity."""
+    rte = S.make_rte(blob8("open", nmu=nmu, nphi=nphi))
+    assert rte.plan_size("nlm") == nmu * nmu
+    y, w = (rte.plan_array(k).astype(np.float64) for k in ("ymat", "wmat"))
+    l = np.arange(nmu)
+    j = l * (l + 1)
+    np.testing.assert_allclose((w.T @ y)[np.ix_(j, j)], np.eye(nmu), atol=1e-5)
+
+
 def test_memory_parameters_follow_the_reference():
     """MAXIG / MAXIC / MAXIV / MAXIDO as RTE._setup_memory sizes them
     (solver.py:2244-2299): adapt_grid_factor x base points, cells 1.5x points,
