@@ -41,6 +41,42 @@ int copy_out(const std::vector<T>& v, void* dst, size_t nbytes, char* err, size_
   if (need) memcpy(dst, v.data(), need);
   return AT3D_OK;
 }
+
+// (options that choose another sweep or transform lay out its arrays)
+int set_option(at3d::State& s, const std::string& k, int32_t value, std::string& err) {
+  if (k == "sweep_general") {
+    s.force_general = value ? 1 : 0;
+    return AT3D_OK;
+  }
+  if (k == "sweep_graph") {
+    s.use_graph = value ? 1 : 0;
+    return AT3D_OK;
+  }
+  if (k == "sweep_ring") {
+    s.use_ring = value < 0 ? 0 : (value > 2 ? 2 : value);
+    return s.use_ring == 2 ? ensure_ring(s, err) : AT3D_OK;
+  }
+  if (k == "render_correct_interpolate") {
+    s.render_correct_interp = value ? 1 : 0;
+    return AT3D_OK;
+  }
+  if (k == "sweep_ring4") return state_set_ring4(s, value != 0, err);
+  if (k == "dense_analysis") {
+    s.dense_analysis = value != 0;
+    const int rc = ensure_dense_analysis(s, err);
+    return rc ? rc : radiance_rows_written(s, err);
+  }
+  if (k == "iteration_graph") {
+    s.use_iter_graph = value ? 1 : 0;
+    return AT3D_OK;
+  }
+  if (k == "max_subgrid_intervals") {
+    s.max_subgrid = value > 0 ? value : 0;
+    return AT3D_OK;
+  }
+  err = "unknown option '" + k + "'";
+  return AT3D_ERR_ARG;
+}
 }  // namespace
 
 extern "C" {
@@ -612,53 +648,16 @@ int at3d_state_set_option(at3d_state* st, const char* key, int32_t value, char* 
     set_err(err, errlen, "null argument");
     return AT3D_ERR_ARG;
   }
-  const std::string k(key);
-  if (k == "sweep_general") {
-    st->s.force_general = value ? 1 : 0;
-    return AT3D_OK;
+  std::string msg;
+  int rc;
+  try {
+    rc = set_option(st->s, key, value, msg);
+  } catch (const std::bad_alloc&) {
+    rc = AT3D_ERR_MEMORY;
+    msg = "out of host memory in an option's arrays";
   }
-  if (k == "sweep_graph") {
-    st->s.use_graph = value ? 1 : 0;
-    return AT3D_OK;
-  }
-  if (k == "sweep_ring") {
-    st->s.use_ring = value < 0 ? 0 : (value > 2 ? 2 : value);
-    if (st->s.use_ring == 2) {
-      std::string e;
-      const int rc = ensure_ring(st->s, e);
-      if (rc) set_err(err, errlen, e.c_str());
-      return rc;
-    }
-    return AT3D_OK;
-  }
-  if (k == "render_correct_interpolate") {
-    st->s.render_correct_interp = value ? 1 : 0;
-    return AT3D_OK;
-  }
-  if (k == "sweep_ring4") {
-    std::string e;
-    const int rc = state_set_ring4(st->s, value != 0, e);
-    if (rc) set_err(err, errlen, e.c_str());
-    return rc;
-  }
-  if (k == "dense_analysis") {
-    st->s.dense_analysis = value != 0;
-    std::string e;
-    int rc = ensure_dense_analysis(st->s, e);
-    if (!rc) rc = radiance_rows_written(st->s, e);
-    if (rc) set_err(err, errlen, e.c_str());
-    return rc;
-  }
-  if (k == "iteration_graph") {
-    st->s.use_iter_graph = value ? 1 : 0;
-    return AT3D_OK;
-  }
-  if (k == "max_subgrid_intervals") {
-    st->s.max_subgrid = value > 0 ? value : 0;
-    return AT3D_OK;
-  }
-  set_err(err, errlen, "unknown option '" + k + "'");
-  return AT3D_ERR_ARG;
+  if (rc) set_err(err, errlen, msg);
+  return rc;
 }
 
 double at3d_state_timing(const at3d_state* st, const char* key) {
