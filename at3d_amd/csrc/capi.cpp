@@ -675,17 +675,19 @@ double at3d_state_timing(const at3d_state* st, const char* key) {
   if (k == "sweep_launches") return s.nsweep_launch;
   if (k == "sweep_kernel") return s.tsum[6];
   if (k == "device_bytes") return (double)s.device_bytes;
-  // a level-ordered sweep (by planes or the ring)
-  if (k == "sweep_ring") return planes_active(s) || ring_active(s) ? 1.0 : 0.0;
+  if (k == "sweep_ring") return ring_active(s) ? 1.0 : 0.0;
   if (k == "sweep_planes") return planes_active(s) ? 1.0 : 0.0;
-  if (k == "sweep_ring_lds")
-    return (double)(planes_active(s) ? s.plane_lds : s.ring_full ? s.ring_lds_full : s.ring_lds);
-  if (k == "sweep_ring_slots") return s.slots;
-  // the grid's ring holds radiances alone, whichever sweep runs
-  if (k == "sweep_ring4") return s.ring_tried ? s.ring4 : ring_wants_radiances_alone(s);
-  if (k == "sweep_ring_full") return s.ring_full;
-  if (k == "sweep_sectors") return s.nsectors;
-  if (k == "sweep_general_points") return s.ngeneral;
+  if (k == "sweep_planes_lds") return s.planes_ok ? (double)s.plane_lds : -1.0;
+  // the ring's layout; none is made before something needs it
+  if (k == "sweep_ring_lds" || k == "sweep_ring_slots" || k == "sweep_ring4" || k == "sweep_ring_full" ||
+      k == "sweep_sectors" || k == "sweep_general_points") {
+    if (!s.ring_ok) return -1.0;
+    if (k == "sweep_ring_lds") return (double)(s.ring_full ? s.ring_lds_full : s.ring_lds);
+    if (k == "sweep_ring_slots") return s.slots;
+    if (k == "sweep_ring4") return s.ring4;
+    if (k == "sweep_ring_full") return s.ring_full;
+    return k == "sweep_sectors" ? s.nsectors : s.ngeneral;
+  }
   if (k == "iters") return s.iters_last;
   if (k == "render") return s.render_ms;
   if (k == "render_rays") return s.render_ray_ms;

@@ -201,24 +201,6 @@ static int ensure_ranks(State& s, std::string& err) {
   return AT3D_OK;
 }
 
-// Whether the ring of this state's grid holds radiances alone: pairs of
-// radiance and source over the five levels that four-point sectors need do
-// not fit in LDS (build_ring_plan, without the layout).
-bool ring_wants_radiances_alone(const State& s) {
-  const Plan& p = *s.plan;
-  if (!p.treeptr.empty()) return false;
-  int slots = 0, nlev = 0;
-  for (int o = 0; o < 8; o++) {
-    if (s.oct_nord[o] <= 0) continue;
-    const std::vector<int32_t>& off = p.oct[o].ring_off;
-    const int n = p.oct[o].ring_nlev;
-    nlev = std::max(nlev, n);
-    for (int L = 0; L <= n && L < (int)off.size(); L++)
-      slots = std::max(slots, off[std::min(n, L + 5)] - off[L]);
-  }
-  return s.force_ring4 || ring_lds_bytes(slots, nlev + 2, 0, 8) > GFX950_LDS_BYTES;
-}
-
 // The level-ordered sweep: each octant's ring order (its levels, with the
 // hemisphere's boundary points as entries of their own), the SH->DO column
 // tiles, the ring sizes, the sectors, and the per-solve step records.  Leaves

@@ -256,7 +256,6 @@ bool planes_active(const State& s);
 int ensure_dense_analysis(State& s, std::string& err);
 int radiance_rows_written(State& s, std::string& err);
 bool ring_active(const State& s);
-bool ring_wants_radiances_alone(const State& s);
 // The ring's layout where it has not been made yet.
 int ensure_ring(State& s, std::string& err);
 

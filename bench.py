@@ -256,9 +256,10 @@ def polarized_leg(cpu_runs):
     out = {"workload": "128x128x64 open cloud, NSTOKES 3, NMU16 NPHI32 L15, solacc 1e-4, "
                        "3 wavelengths (0.47 0.66 0.86 um), 9 views of 128x128 I/Q/U",
            "npts": rtes[0].plan_size("npts"),
-           "sweep": ("plane-ordered ({:.0f} KB of LDS)" if rtes[0].timing("sweep_planes") else
-                     "level-ordered, ring of radiances ({:.0f} KB of LDS)" if rtes[0].timing("sweep_ring4") else
-                     "level-ordered ({:.0f} KB of LDS)").format(rtes[0].timing("sweep_ring_lds") / 1024)
+           "sweep": "plane-ordered ({:.0f} KB of LDS)".format(rtes[0].timing("sweep_planes_lds") / 1024)
+           if rtes[0].timing("sweep_planes") else
+           ("level-ordered, ring of radiances ({:.0f} KB of LDS)" if rtes[0].timing("sweep_ring4") else
+            "level-ordered ({:.0f} KB of LDS)").format(rtes[0].timing("sweep_ring_lds") / 1024)
            if rtes[0].timing("sweep_ring") else "point-ordered",
            "iterations": [r.num_iterations for r in rtes], "solve_wall_s": wall,
            "solves_per_s": len(ws) / wall, "render_wall_s": render_s,
@@ -543,8 +544,10 @@ def main():
                      "GB/s": sweep_bytes / 2 / ms_launch / 1e6,
                      "level_ordered": bool(rte.timing("sweep_ring")),
                      "plane_ordered": bool(rte.timing("sweep_planes")),
-                     "lds_bytes": int(rte.timing("sweep_ring_lds")),
-                     "multi_cell_points": int(rte.timing("sweep_general_points"))}
+                     "lds_bytes": int(max(rte.timing("sweep_planes_lds" if rte.timing("sweep_planes") else
+                                                     "sweep_ring_lds"), 0))}
+    if rte.timing("sweep_ring"):
+        kern["sweep"]["multi_cell_points"] = int(rte.timing("sweep_general_points"))
     # the transforms on the terms that can be nonzero (each point's source
     # truncation NS for SH->DO, radiance truncation NR for DO->SH): bytes one
     # read or write of those terms and of NANG values per point; the flops of a

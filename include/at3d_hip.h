@@ -364,11 +364,15 @@ int at3d_state_set_option(at3d_state* st, const char* key, int32_t value, char* 
  * device allocations); of the
  * last render call "render" (direction source and rays) and "render_rays"
  * (the ray kernel alone); of the last gradient call "gradient" and
- * "adjoint_rays" (the adjoint ray kernel alone).  The sweep's layout: "sweep_ring"
- * (1 when the level-ordered sweep runs), "sweep_ring_lds" (its LDS bytes),
+ * "adjoint_rays" (the adjoint ray kernel alone).  The sweep that the options
+ * select: "sweep_planes" (1: the plane-ordered one), "sweep_ring" (1: the
+ * level-ordered ring), neither: point by point.  "sweep_planes_lds": the plane
+ * sweep's LDS bytes.  The ring's layout: "sweep_ring_lds" (its LDS bytes),
  * "sweep_ring_slots", "sweep_ring4" (1 for 4-byte slots), "sweep_ring_full" (1 when
- * every column takes the full instantiation), "sweep_sectors".
- * Returns a negative value for unknown keys. */
+ * every column takes the full instantiation), "sweep_sectors",
+ * "sweep_general_points" (points, over the ordinates, of the multi-cell trace).
+ * Returns a negative value for unknown keys, and for the layout of a sweep that
+ * the state does not hold. */
 double at3d_state_timing(const at3d_state* st, const char* key);
 
 #ifdef __cplusplus

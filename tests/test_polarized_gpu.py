@@ -131,9 +131,8 @@ def test_a1_only_polarized_equals_scalar():
 
 @pytest.mark.parametrize("bc", ["open", "periodic"])
 def test_polarized_point_ordered_sweep(ref, bc):
-    """Grids whose rings do not fit in LDS sweep point by point: the same I,
-    Q, U (the one-cell path bit for bit against the general trace) and the
-    reference's converged fields."""
+    """Point by point, here from per-ordinate records: the same I, Q, U (bit for
+    bit against the general trace) and the reference's converged fields."""
     w = pol_blob(bc=bc)
     a = S.make_rte(w)
     a.set_option("sweep_ring", 0)
@@ -175,15 +174,21 @@ def test_polarized_ring_of_radiances(bc):
 def test_polarized_large_grid_takes_ring_of_radiances():
     """A 96 x 96 x 64 polarized grid (16 x 32 ordinates), whose ring of
     (radiance, source) pairs needs about 200 KB of LDS, takes the 4-byte ring
-    (about 100 KB) by itself; two iterations of it agree with the
+    (about 100 KB) by itself where it goes by the ring; two iterations of it, and
+    of the planes that it goes by unless told otherwise, agree with the
     point-ordered sweep (rel L2 <= 2e-6 for I, Q, U)."""
     w = S.polarized_cloud_field(nx=96, ny=96, nz=64, seed=2)
+    p = S.make_rte(w, max_total_mb=60000, adapt_grid_factor=1.0)
+    p.solve(2, verbose=False)
+    assert p.timing("sweep_planes") == 1.0 and p.timing("sweep_ring") == 0.0
     a = S.make_rte(w, max_total_mb=60000, adapt_grid_factor=1.0)
+    a.set_option("sweep_ring", 2)
     a.solve(2, verbose=False)
-    assert a.timing("sweep_ring") == 1.0 and a.timing("sweep_ring4") == 1.0
+    assert a.timing("sweep_planes") == 0.0 and a.timing("sweep_ring") == 1.0 and a.timing("sweep_ring4") == 1.0
     b = S.make_rte(w, max_total_mb=60000, adapt_grid_factor=1.0)
     b.set_option("sweep_ring", 0)
     b.solve(2, verbose=False)
-    got, want = a.state_array("source"), b.state_array("source")
-    for k in range(3):
-        assert rel_l2(got[k], want[k]) < 2e-6, k
+    want = b.state_array("source")
+    for got in (a.state_array("source"), p.state_array("source")):
+        for k in range(3):
+            assert rel_l2(got[k], want[k]) < 2e-6, k

@@ -33,7 +33,7 @@ def _ref_dense(ref, st, which):
                          ids=["blob8_open", "cloud12_two_species", "blob8_open_l15", "cloud16_l15"])
 def test_sh_to_do_gemm_matches_numpy(make):
     """The two-species scene mixes points of 9 and of many source terms, so
-    the level-ordered transform's K extent varies from tile to tile."""
+    the plane-ordered transform's K extent varies from tile to tile."""
     w = make()
     rte = S.make_rte(w)
     rte.solve(0)
@@ -107,15 +107,23 @@ def test_converged_solution_matches_reference(ref, make):
     assert rel_l2(rte.state_array("fluxes"), st.fluxes[:, :st.npts]) < 1e-4
 
 
-@pytest.mark.parametrize("make", [lambda: blob8("periodic"), lambda: blob8("open"), cloud_small],
-                         ids=["blob8_periodic", "blob8_open", "cloud12_two_species"])
+def _past_the_records():
+    # 43560 points: an ordinate's radiances do not fit in LDS, so the point
+    # order traces in every sweep, one-cell points by the analytic path
+    return S.cloud_field(nx=40, ny=33, nz=33, dx=0.05, dz=0.03, z0=0.3, seed=3, nmu=4, nphi=8)
+
+
+@pytest.mark.parametrize("make", [lambda: blob8("periodic"), lambda: blob8("open"), cloud_small, _past_the_records],
+                         ids=["blob8_periodic", "blob8_open", "cloud12_two_species", "cloud40x33x33"])
 def test_fast_sweep_path_bit_identical_to_general_trace(make):
-    """The point-ordered sweep's analytic one-cell path must reproduce the
-    general trace exactly."""
+    """The point-ordered sweep must reproduce the general trace exactly: from
+    records on small grids, by its analytic one-cell path past 40960 points
+    (where its iterations do not run from graphs)."""
     w = make()
     a = S.make_rte(w)
     a.set_option("sweep_ring", 0)
     a.solve(3, verbose=False)
+    assert a.timing("iteration_graph_active") == (1.0 if a.state_size("npts") <= 40960 else 0.0)
     b = S.make_rte(w)
     b.set_option("sweep_general", 1)
     b.solve(3, verbose=False)
@@ -194,29 +202,40 @@ def test_ring_of_radiances_matches_ring_of_pairs(make):
 
 def test_chain_levels_take_the_point_ordered_sweep():
     """Periodic grids, whose dependency levels are chains of a point or two,
-    sweep point by point by default (faster there); open grids keep the
-    level-ordered ring; option 2 forces the ring."""
+    sweep point by point by default (faster there); open grids go by planes,
+    uneven ones keep the level-ordered ring; option 2 forces the ring.  A ring
+    that was not laid out has no layout to report."""
     a = S.make_rte(blob8("periodic"))
     a.solve(2, verbose=False)
-    assert a.timing("sweep_ring") == 0.0
+    assert a.timing("sweep_ring") == 0.0 and a.timing("sweep_planes") == 0.0
+    assert a.timing("sweep_ring4") == -1.0 and a.timing("sweep_general_points") == -1.0
     a.set_option("sweep_ring", 2)
-    assert a.timing("sweep_ring") == 1.0
+    assert a.timing("sweep_ring") == 1.0 and a.timing("sweep_ring4") == 0.0
     b = S.make_rte(blob8("open"))
     b.solve(2, verbose=False)
-    assert b.timing("sweep_ring") == 1.0
+    assert b.timing("sweep_ring") == 0.0 and b.timing("sweep_planes") == 1.0
+    b.set_option("sweep_ring", 2)
+    assert b.timing("sweep_ring") == 1.0 and b.timing("sweep_planes") == 0.0
+    w = blob8("open")
+    w.z = (0.3 * (np.arange(8) / 7.0) ** 2.5).astype(np.float32)
+    c = S.make_rte(w)
+    c.solve(2, verbose=False)
+    assert c.timing("sweep_ring") == 1.0 and c.timing("sweep_planes") == 0.0
 
 
 def test_sweep_graph_replay_bit_identical_to_direct_launches():
-    """The point-ordered sweep replayed from a HIP graph against direct launches
-    (the level-ordered sweep is always launched directly)."""
+    """The point-ordered sweep that traces in every sweep, replayed from a HIP
+    graph, against direct launches (the other sweeps are launched directly, or
+    run in the graphs of whole iterations)."""
     w = cloud_small()
     a = S.make_rte(w)
-    a.set_option("sweep_ring", 0)
+    a.set_option("sweep_general", 1)
     a.solve(4, verbose=False)
     b = S.make_rte(w)
-    b.set_option("sweep_ring", 0)
+    b.set_option("sweep_general", 1)
     b.set_option("sweep_graph", 0)
     b.solve(4, verbose=False)
+    assert a.timing("iteration_graph_active") == 0.0 and b.timing("iteration_graph_active") == 0.0
     assert np.array_equal(a.state_array("do_radiance"), b.state_array("do_radiance"))
     assert np.array_equal(a.state_array("source"), b.state_array("source"))
     assert a.num_iterations == b.num_iterations
@@ -246,8 +265,10 @@ def test_wide_open_grid_keeps_every_step_in_its_class():
     from device memory."""
     w = S.serve_medium((96, 96, 48), 16, 32, 0.86, 1)
     rte = S.make_rte(w)
+    rte.set_option("sweep_ring", 2)
     rte.solve(0, verbose=False)
-    assert rte.timing("sweep_ring") == 1.0
+    assert rte.timing("sweep_ring") == 1.0 and rte.timing("sweep_planes") == 0.0
+    assert rte.timing("sweep_ring_full") == 1.0
     assert rte.timing("sweep_general_points") == 0
     # the class tolerance keeps the results: three iterations against the
     # point-ordered FP64-geometry sweep.  The steps of one class here differ
