@@ -691,6 +691,8 @@ double at3d_state_timing(const at3d_state* st, const char* key) {
   if (k == "iters") return s.iters_last;
   if (k == "render") return s.render_ms;
   if (k == "render_rays") return s.render_ray_ms;
+  if (k == "render_listed") return s.render_listed;
+  if (k == "gradient_listed") return s.grad_listed;
   if (k == "iteration_graph_active") return s.last_solve_graph ? 1.0 : 0.0;
   if (k == "adjoint_rays") return s.adjoint_ms;
   if (k == "gradient") return s.grad_ms;

@@ -292,7 +292,8 @@ int state_levis_gradient(State& s, const at3d_deriv_desc& dd, int64_t nrays, con
   const size_t o_dirs = carve((size_t)ndir * 16), o_dpt = carve(g.dphasetab.size() * 4);
   // rays with directions of their own: the source and GRAD8 at the points
   // around each ray's path alone (the Jacobian takes the full tables)
-  bool pairs = njac == 0 && pair_source_pays(s, nrays, ndir);
+  const bool listed = njac == 0 && pair_source_pays(s, nrays, ndir);
+  bool pairs = listed;
   const int cap = pair_cap(p);
   const size_t o_cnt = carve(pairs ? (size_t)nrays * 4 : 0), o_over = carve(4);
   const size_t o_list = carve(pairs ? (size_t)nrays * cap * 4 : 0);
@@ -650,6 +651,7 @@ int state_levis_gradient(State& s, const at3d_deriv_desc& dd, int64_t nrays, con
   float ms = 0.f;
   (void)hipEventElapsedTime(&ms, s.ev[6], s.ev[7]);
   s.grad_ms = ms;
+  s.grad_listed = pairs ? 1 : listed ? 2 : 0;
   (void)hipEventElapsedTime(&ms, s.ev_ray[0], s.ev_ray[1]);
   s.adjoint_ms = ms;
   if (ef) {

@@ -407,6 +407,7 @@ static int render_impl(State& s, int64_t nrays, const float* x, const float* y, 
   float ms = 0.f;
   (void)hipEventElapsedTime(&ms, s.ev[6], s.ev[7]);
   s.render_ms = ms;
+  s.render_listed = pairs ? 1 : dense ? 2 : 0;
   (void)hipEventElapsedTime(&ms, s.ev_ray[0], s.ev_ray[1]);
   s.render_ray_ms = ms;
   if (ef) {

@@ -179,6 +179,9 @@ struct State {
   int max_subgrid = 0;     // extra sub-step intervals a gradient ray may record
   double grad_ms = 0.0;
   double render_ms = 0.0;
+  // the source the last render / gradient call read: 0 every point's, 1 the listed
+  // points' alone, 2 every point's since a ray passed its list
+  int render_listed = 0, grad_listed = 0;
   double render_ray_ms = 0.0;   // k_render alone in the last render call
   double adjoint_ms = 0.0;      // k_adjoint_rays alone in the last gradient call
 };

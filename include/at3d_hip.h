@@ -364,7 +364,10 @@ int at3d_state_set_option(at3d_state* st, const char* key, int32_t value, char* 
  * device allocations); of the
  * last render call "render" (direction source and rays) and "render_rays"
  * (the ray kernel alone); of the last gradient call "gradient" and
- * "adjoint_rays" (the adjoint ray kernel alone).  The sweep that the options
+ * "adjoint_rays" (the adjoint ray kernel alone); "render_listed" and
+ * "gradient_listed": the direction source the call read was made at every point
+ * (0), at the points around the rays' paths alone (1), or at every point because
+ * a ray crossed more cells than its list holds (2).  The sweep that the options
  * select: "sweep_planes" (1: the plane-ordered one), "sweep_ring" (1: the
  * level-ordered ring), neither: point by point.  "sweep_planes_lds": the plane
  * sweep's LDS bytes.  The ring's layout: "sweep_ring_lds" (its LDS bytes),
