@@ -69,10 +69,12 @@ def test_ray_past_its_list_takes_the_full_table():
 
 
 @pytest.mark.filterwarnings("ignore")
-@pytest.mark.parametrize("correct", [1, 0])
+@pytest.mark.parametrize("correct", [True, False])
 def test_refined_grid_listed_points_match_full_table(correct):
+    """Also where a cell starts with the values the ray left the last one with,
+    which differ from its own on a face between cells of two sizes."""
     w, rte = _refined()
-    rte.set_option("render_correct_interpolate", correct)
+    rte._correctinterpolate = correct
     n = 1500
     rays = interior_rays(w, n, seed=5)
     a = rte.integrate_to_sensor(dict(rays))["I"]
