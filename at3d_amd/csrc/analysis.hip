@@ -20,7 +20,9 @@
 // sign, so both components' products share the operands.
 //
 // Bound by the round trips of a tile with one workgroup on a CU (its LDS holds
-// 64 columns' sums and coefficients), at about half the rate of a large copy.
+// 64 columns' sums and coefficients), at about half the rate of a large copy.  Q
+// and U with more than 8 zenith angles spill 2 vector registers up to 31 azimuths,
+// 11 from 32 on.
 // NMU 16, an iteration, the dense product before: 64 x 64 x 40 81 us for 240,
 // 96 x 96 x 48 216 for 645, 128 x 128 x 64 I 0.51 ms for 1.48 and Q with U 1.52
 // for 5.40.  Tried: the same sums a lane a point from scalar tables, 170 us at

@@ -189,20 +189,26 @@ void launch_sweep_preset(hipStream_t st, const SweepArgs& a, bool up, int col0, 
 // One workgroup per ordinate column col0 .. col0+ncol-1, all levels of its octant.
 void launch_sweep_columns(hipStream_t st, const SweepArgs& a, int col0, int ncol);
 // ---- sweep_planes.hip: plane-ordered sweep of open base grids -------------
-// Per axis t (0: z, 1: x, 2: y) the planes across it, in ascending coordinate:
-// within plane k a point's natural index is s = y + ny x (z), z + nz y (x) or
-// z + nz x (y); the source rows of an axis's columns hold plane k at k * M ..
-// (k + 1) * M (M points a plane), within a plane in the order of pidx.
+// Per axis t (0: z, 1: x, 2: y) the N planes across it, in ascending coordinate:
+// within a plane a point's natural index is s = y + ny x (z), z + nz y (x) or
+// z + nz x (y), rows of na = ny, nz or nz points.  A plane goes in strips of sb[t]
+// rows (one strip where sb[t] is all of them, the last one of what is left).  The
+// source rows of an axis's columns hold strip after strip, a strip of M points
+// from row b0 on plane by plane: plane k of it from na * b0 * N + k * M, in the
+// order of pidx, whose places count from the strip's first point.  `ext` holds whole
+// planes.
 struct PlaneArgs {
   const int8_t* col_type = nullptr;   // [ncols] axis; + 4: an open side's plane is swept by the other
                                       // horizontal axis, not by z
-  const uint16_t* pidx = nullptr;     // [3][npts] natural index of each position of a source row
+  const uint16_t* pidx = nullptr;     // [3][npts] place in its strip's plane of each position of a source row
   const float* ext = nullptr;         // [3][npts] extinction, plane by plane, natural order
   double dx = 0, dy = 0;              // horizontal spacings
   int sb[3] = {};                     // rows a strip of each axis's planes
 };
 // Largest plane in one piece, and largest strip of others: four and three points
-// a thread of 1024, what their registers hold (strips of four spill 52).
+// a thread of 1024.  Their vector registers hold that but for one or two (strips of
+// four spill 52); of the scalar ones 25 to 66, and 117 in strips, go to vector
+// registers' lanes.
 constexpr int PLANE_POINTS_MAX = 4096, PLANE_STRIP_MAX = 3072;
 // Planes (strips of planes) of mz points across z and ms across x or y.
 int sweep_planes_max_lds(int mz, int ms, bool strips, size_t lds);

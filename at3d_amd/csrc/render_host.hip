@@ -197,8 +197,11 @@ int pair_cap(const Plan& p) {
 // few rays a direction.  The full table takes 23 ps a point and direction with
 // its passes over memory; listing takes a traversal of its own, bound by latency
 // (1.4 us for every plane of the grid a ray can cross), and 0.2 ns a listed
-// point, of which a ray has about 1.6 a plane (both measured with one camera over
-// 64 x 64 x 40 points: 14 ms against 0.42 at 61 x 61 pixels).
+// point, of which a ray has about 1.6 a plane (the constants come from one camera
+// over 64 x 64 x 40 points: 14 ms against 0.42 at 61 x 61 pixels).  Both ways timed
+// for one camera of 2 x 2 to 90 x 90 pixels over eight grids from 12 x 12 x 10 to
+// 96 x 96 x 48, NMU 8 to 16: the rule takes the slower way at four of 51, all next to
+// the line and by 9 % at most (40 x 36 x 30, 169 directions: 0.49 ms for 0.45).
 bool pair_source_pays(const State& s, int64_t nrays, int ndir) {
   const Plan& p = *s.plan;
   const double planes = p.nx1 + p.ny1 + p.nz;

@@ -24,10 +24,12 @@
 // x ordinate, runs of nz for y, and four planes at a time (16 bytes a point) for
 // z.
 //
-// Bound by the vector units' issue: some 55 instructions a point, most of them
-// the transmission and source weights of cell_coefs, which the ring read from
-// records (8 bytes a point and ordinate each iteration, and a pass of its own
-// per solve to make them).  Per hemisphere, against k_sweep_ring: 64 x 64 x 40,
+// No one unit bounds it: at 64 x 64 x 40 the vector units issue 80 instructions a
+// point (the transmission and source weights of cell_coefs and the interpolation,
+// and the moves of scalars spilled to vector lanes) half of the time, the LDS is in use
+// for 53 % of it, two thirds of that in bank conflicts of the 16-byte points, and a
+// wavefront waits half of its life, mostly at the two barriers a plane.  Per
+// hemisphere, against k_sweep_ring: 64 x 64 x 40,
 // 142 ordinates 138 against 253 us; 32 x 32 x 32, 56 ordinates 37 against 92;
 // 48^3, cold 84 against 156 and no records pass (730 us a solve).  Plane order
 // also feeds SH->DO longer runs of one class: 128 against 153 us at 64 x 64 x 40.
