@@ -5,18 +5,20 @@
 //   SH -> DO transform   (SH_TO_DO_UNPOL :2928) MFMA GEMM      transforms.hip
 //   downwelling sweeps, Lambertian surface, upwelling sweeps
 //                        (PATH_INTEGRATION :1836, BACK_INT_GRID3D_UNPOL :3695)
-//                        one workgroup per ordinate over per-solve step records,
-//                        replayed from a HIP graph                               sweep.hip
-//   DO -> SH transform   (DO_TO_SH_UNPOL :3164) MFMA GEMM      transforms.hip
+//                        one workgroup per ordinate: by planes     sweep_planes.hip,
+//                        from per-ordinate records                sweep_chain.hip,
+//                        by the ring or point by point            sweep.hip
+//   DO -> SH transform   (DO_TO_SH_UNPOL :3164) by factors     analysis.hip,
+//                        or MFMA GEMM                          transforms.hip
 //   source function      (COMPUTE_SOURCE :967)                 source.hip
 //   criterion            (CALC_ACCEL_SOLCRIT shdom_nompi.f:317) host, single precision
 //   acceleration         (ACCELERATE_SOLUTION :1807)           source.hip
 //
 // Device layouts: SH fields [point][ld] (ld = nlm rounded up to 64); DO fields
 // ordinate-major [ldo][nptsp] with the ordinates grouped by octant (ldo = nang
-// rounded up to 64, nptsp = points rounded up to 64, padding zero).  With the
-// level-ordered sweep the DO source rows are in their octant's position order
-// (boundary points, then sweep levels) and the DO radiance rows by point.
+// rounded up to 64, nptsp = points rounded up to 64, padding zero).  The DO source
+// rows are in the order of the sweep that reads them (plane by plane, the ring's
+// levels, or by point) and the DO radiance rows by point.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdio.h>
@@ -203,7 +205,7 @@ static int ensure_ranks(State& s, std::string& err) {
 
 // The level-ordered sweep: each octant's ring order (its levels, with the
 // hemisphere's boundary points as entries of their own), the SH->DO column
-// tiles, the ring sizes, the sectors, and the per-solve step records.  Leaves
+// tiles, the ring sizes, the sectors, and the state's step records.  Leaves
 // ring_ok false (and the point-ordered sweep in use) when the rings do not fit
 // in LDS or the records do not fit in memory.
 static int setup_ring(const Plan& p, State& s, std::string& err) {

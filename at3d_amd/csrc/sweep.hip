@@ -14,9 +14,9 @@
 // plane-ordered sweep (sweep_planes.hip) or whose planes do not fit in LDS in
 // strips.
 // Everything about a one-cell
-// characteristic that stays fixed during a solve (face points, bilinear
-// weights, transmission, the source-integral coefficients) is computed once
-// per solve by k_sweep_records and stored in level order, so a level is read
+// characteristic that stays fixed in a state (face points, bilinear
+// weights, the face's extinction) is computed once
+// per state by k_sweep_records and stored in level order, so a level is read
 // as one contiguous block.  The radiances and source values of the last
 // RING_LEVELS levels and of the boundary points live in LDS; a level then
 // costs LDS gathers, a few FMAs and a barrier that waits for LDS traffic only,

@@ -29,9 +29,9 @@
 // and the moves of scalars spilled to vector lanes) half of the time, the LDS is in use
 // for 53 % of it, two thirds of that in bank conflicts of the 16-byte points, and a
 // wavefront waits half of its life, mostly at the two barriers a plane.  Per
-// hemisphere, against k_sweep_ring: 64 x 64 x 40,
-// 142 ordinates 138 against 253 us; 32 x 32 x 32, 56 ordinates 37 against 92;
-// 48^3, cold 84 against 156 and no records pass (730 us a solve).  Plane order
+// hemisphere, against k_sweep_ring: 64 x 64 x 40, 177 ordinates 138 against 253 us;
+// 32 x 32 x 32, 45 ordinates 37 against 92;
+// 48 x 48 x 32, cold 84 against 156 and no records pass (730 us a solve).  Plane order
 // also feeds SH->DO longer runs of one class: 128 against 153 us at 64 x 64 x 40.
 //
 // Planes past PLANE_POINTS_MAX go in strips of rows, one after the other in the
@@ -39,7 +39,7 @@
 // only its last row, whose radiances and sources stay in LDS (8 bytes a line and
 // plane).  More points a thread instead spill registers (96 x 96 planes, ten a
 // thread: 1012 us a hemisphere; 128 x 128, 16: 16.8 ms).  Against the ring:
-// 96 x 96 x 48, 142 ordinates, 405 us for 984; 128 x 128 x 64 with three Stokes
+// 96 x 96 x 48, 177 ordinates, 405 us for 984; 128 x 128 x 64 with three Stokes
 // components 2.0 ms for 5.77.
 #include <hip/hip_runtime.h>
 

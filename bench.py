@@ -539,7 +539,9 @@ def main():
     # pass also holds the surface boundary kernel
     ms_launch = ksum["sweep_kernel"] / n_it / 2 if ksum["sweep_kernel"] > 0 else ms_pass / 2
     kern["sweep"] = {"ms_per_pass": ms_pass, "launches_per_pass": 2,
-                     "dependency_levels": sweep_levels,
+                     # (planes: as many as the longest axis has, at most)
+                     "dependency_levels": max(rte.plan_size(k) for k in ("nx", "ny", "nz"))
+                     if rte.timing("sweep_planes") else sweep_levels,
                      "ms_per_launch": ms_launch, "bytes_per_launch": sweep_bytes / 2,
                      "GB/s": sweep_bytes / 2 / ms_launch / 1e6,
                      "level_ordered": bool(rte.timing("sweep_ring")),

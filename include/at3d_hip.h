@@ -334,24 +334,31 @@ int at3d_levis_gradient_jacobian(at3d_state* st, const at3d_deriv_desc* deriv, i
 /* Engine options of a state.  "sweep_general" (0/1): route every grid point
  * through the general multi-cell characteristic trace of the point-ordered
  * sweep (bit-identical to its analytic one-cell path; for tests).
- * "sweep_ring" (0/1/2, default 1): use the level-ordered sweep with per-solve
- * step records and an LDS ring when the ring fits (else the point-ordered
- * sweep); 1 leaves grids whose dependency levels are chains (under four
- * points a level, as periodic grids have) to the point-ordered sweep, which
- * is faster there; 2 takes the ring wherever it fits.  "sweep_ring4" (0/1, default 0): lay the ring out with 4-byte
+ * "sweep_ring" (0/1/2, default 1): which sweep an open or periodic base grid
+ * takes.  1: by planes, where every ordinate goes by one axis through all layers
+ * of an open grid and strips of planes and the ring both fit in LDS; else the
+ * level-ordered ring with step records, where it fits and the dependency levels
+ * are no chains (under four points a level, as periodic grids have); else point
+ * by point.  2: the ring wherever it fits, laid out when the option is set.  0:
+ * point by point.  Planes and ring step in single precision, point by point in
+ * double; a grid whose ring does not fit goes point by point, never by planes.
+ * The point order keeps per-ordinate records up to 40960 points and traces in
+ * every sweep past them.  "sweep_ring4" (0/1, default 0): lay the ring out with 4-byte
  * slots (radiances alone; the sources are read from the state's arrays) even
  * where (radiance, source) pairs fit; grids whose pairs exceed LDS take it by
  * themselves (for tests; rebuilds the layout and drops the captured graphs).
- * "sweep_graph" (0/1): replay the sweep launches from a HIP graph.
+ * "sweep_graph" (0/1): replay the launches of the sweep that traces in every
+ * sweep from a HIP graph.
+ * "dense_analysis" (0/1, default 0): DO->SH as one dense product also where the
+ * angle set (NMU <= 16, at most 39 azimuths) goes by azimuth and Legendre sums.
  * "render_correct_interpolate" (0/1, default 1): RENDER's CORRECTINTERPOLATE
  * (shdomsub2.f:2562); 0 starts each cell after a ray's first with the source
  * and extinction it left the previous cell with.
  * "iteration_graph" (0/1, default 1): run a solve's iterations from captured
  * HIP graphs of four iterations each under device control (the convergence
  * test, FIXSH and the acceleration on the device; the host reads the control
- * block once per four iterations) when the level-ordered sweep is in use; 0,
- * verbose, or the point-ordered sweep runs them one by one with the host
- * deciding after each.
+ * block once per four iterations); 0, verbose, cell splitting, or the sweep that
+ * traces in every sweep runs them one by one with the host deciding after each.
  * "max_subgrid_intervals": sub-step intervals one gradient ray may record.
  * No counterpart in the reference. */
 int at3d_state_set_option(at3d_state* st, const char* key, int32_t value, char* err,
